@@ -301,6 +301,11 @@ hipError_t launch_ref_f32_group(const void* x, int xkind, int64_t m, int64_t k, 
                                 const int64_t* n, const float* scale, void* const* y, int count, int ykind,
                                 hipStream_t st, int xf = 0, const RefXf* t = nullptr);
 
+// many token rows through the f32 matrix instructions (btl_mm32.hip): the
+// shapes of the staged form; g.wg_begin is not read
+hipError_t launch_ref_mm(const void* x, int xkind, int64_t m, int64_t k, const RefGroup& g, int ykind,
+                         hipStream_t st);
+
 hipError_t launch_generic_i8(const int8_t* q, const float* xs, int64_t m, int64_t k,
                              const uint8_t* w, int64_t n, float sw, void* y, int ykind,
                              int32_t* acc_out, hipStream_t st);

@@ -3019,6 +3019,12 @@ hipError_t launch_ref_f32_group(const void* x, int xkind, int64_t m, int64_t k, 
         b += (int)((n[i] + rows - 1) / rows);
     }
     g.wg_begin[count] = b;
+    // from 8 token rows and 65536 outputs on the f32 matrix instructions are
+    // faster (us, this form / that one: q|k|v at m = 8 17 / 20, 16 30 / 26, 32 55
+    // / 33; down at m = 8 51 / 59, 16 100 / 77; gate|up at m = 8 61 / 52, 16 118 /
+    // 76): below them a 16-token tile is mostly padding
+    if (xf == 0 && m >= 8 && m * n_total >= 65536)
+        return launch_ref_mm(x, xkind, m, k, g, ykind, st);
     // two token rows per workgroup from m = 2 on (the weight chunk's read and
     // coefficient lookup shared; x of both rows in LDS: at most 2 x 64 KB)
     const int tr = m >= 2 ? 2 : 1;

@@ -679,6 +679,39 @@ def test_linear_f32_ref_staged_form(m, k, n, xdt, ydt):
         assert_bf16_matches(y, yr)
 
 
+# many token rows: the f32 matrix form.  The sizes reach each of its four tile
+# forms (1 x 1 and 1 x 2 blocks of 16 with four chains a wave, 2 x 2 with four
+# and with eight), with ragged token and row tiles, a group of layers, fewer
+# 32-input blocks than are in flight (k = 64) and a remainder of them (k = 320)
+REF_MM_CASES = [(17, 192, (4000,)), (17, 64, (4000, 33)), (33, 320, (5000,)), (65, 64, (4968, 33)),
+                (65, 4096, (1100,)), (128, 320, (8000,)), (100, 64, (8190, 17, 33)), (8, 128, (8192,))]
+
+
+@pytest.mark.parametrize("m,k,ns", REF_MM_CASES)
+@pytest.mark.parametrize("xdt,ydt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16)])
+def test_linear_f32_ref_matrix_form(m, k, ns, xdt, ydt):
+    print("f32 ref matrix form", m, k, ns, xdt, flush=True)
+    rng = np.random.default_rng(m * 7 + k + ns[0])
+    x = (rng.standard_normal((m, k)) * np.exp2(rng.integers(-20, 20, (m, k)))).astype(np.float32)
+    x[1] = rng.standard_normal(k) * 1e-39           # subnormal inputs and sums
+    x[2, 3], x[3, 5] = np.inf, np.nan               # only their own rows turn NaN
+    x[4] = rng.standard_normal(k) * 3e37            # partial sums overflow
+    layers = [(random_codes(n, k, seed=k + n, p3=0.1), np.float32(0.0173 + i), n) for i, n in enumerate(ns)]
+    pts = [bl.PackedTensor(torch.from_numpy(wb).to(DEV), float(sw), (n, k), DEV) for wb, sw, n in layers]
+    xt = to_dev(x, xdt)
+    ys = bl.linear_group(pts, xt, out_dtype=ydt, mode="f32_ref")
+    for y, (wb, sw, n) in zip(ys, layers):
+        yr = orc.forward_f32(host_x(xt), wb, n, sw)
+        nan = np.isnan(yr)
+        assert nan[2:4].any() and not nan[[0, 1]].any()
+        assert np.array_equal(np.isnan(y.float().cpu().numpy()), nan)
+        y, yr = torch.where(torch.from_numpy(nan).to(DEV), 0, y), np.where(nan, 0, yr).astype(np.float32)
+        if ydt == torch.float32:
+            assert_f32_identical(y, yr)
+        else:
+            assert_bf16_matches(y, yr)
+
+
 # special inputs in the reference's order: subnormal inputs and partial sums
 # (fma keeps them), sums that overflow to inf, inf inputs (times a zero
 # coefficient: NaN) and a NaN input; staged (k % 64 == 0) and general forms

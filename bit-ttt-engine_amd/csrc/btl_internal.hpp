@@ -441,5 +441,12 @@ hipError_t launch_rmsnorm_f32(const float* h, const float* delta, float* h_out, 
                               int64_t k, float* y, hipStream_t st);
 hipError_t launch_dense_gemv(const void* w, int wkind, int64_t n, int64_t k, const float* x, int64_t m, float* y,
                              hipStream_t st);
+// several token rows through the f32 matrix instructions (btl_mm32.hip), the
+// same sums; k <= kDenseMmMaxK (32 rows' byte offsets in 31 bits) and at most
+// kDenseMmMaxTiles tiles of 16 x 16 outputs (512 threads each, under 2^32)
+constexpr int64_t kDenseMmMaxK = 1 << 22;
+constexpr int64_t kDenseMmMaxTiles = 1 << 22;
+hipError_t launch_dense_mm(const void* w, int wkind, int64_t n, int64_t k, const float* x, int64_t m, float* y,
+                           hipStream_t st);
 
 }  // namespace btl

@@ -15,6 +15,8 @@
 // Kernels:
 //   k_ref_mm    BTL_ACT_F32_REF of many token rows (BitLinearCpu::forward,
 //               src/kernels/cpu.rs:86-123: eight chains per output)
+//   k_dense_mm  btl_dense_linear of several token rows (candle_nn::Linear,
+//               src/model/llama.rs:129-141; src/layers/adaptive_linear.rs:131-160)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -285,6 +287,278 @@ hipError_t launch_ref_mm(const void* x, int xkind, int64_t m, int64_t k, const R
     BTL_REF_MM(XK_BF16, YK_F32)
     BTL_REF_MM(XK_BF16, YK_BF16)
 #undef BTL_REF_MM
+    return hipErrorInvalidValue;
+}
+
+// ---------------------------------------------------------------------------
+// k_dense_mm
+// ---------------------------------------------------------------------------
+// btl_dense_linear of several token rows: lane l of 64 (a chain) folds the
+// 4-element chunks l, l + 64, ... of a row in element order, then the chains
+// are added in the butterfly's order (xor 32, 16, 8, 4, 2, 1).  One
+// v_mfma_f32_16x16x1_f32 advances four chains of 16 tokens x 16 weight rows by
+// one element: lane 16 c + r holds the element of chain c's chunk for token
+// (weight row) r, so the 16 bytes of a chunk feed four of them and nothing is
+// exchanged between lanes.  Wave s of eight holds the chains 4 s .. 4 s + 3 and
+// 32 + 4 s .. 35 + 4 s of a tile of 16 TB tokens x 16 NB rows (32 TB NB
+// accumulator registers); the first level of the butterfly is then in its
+// registers, the rest in LDS after the main loop.
+//
+// The operands go through LDS: with direct loads the lanes of a quarter wave
+// read 16 different rows, which the address unit takes one line per lane (128
+// tokens x 5632 rows, k = 2048: 63 us, 45 with the copies, whose consecutive
+// lanes read consecutive bytes).  A wave copies and reads only its own chains,
+// so the main loop has no barrier, two stages of 256 elements.
+//
+// What bounds it: the f32 matrix rate from about 64 token rows, below that the
+// weights.  us, k_dense_gemv (which reads the weights again for every token
+// row) -> now: n = 5632, k = 2048, f32: m = 2 15 -> 12, 16 80 -> 14, 128 711 ->
+// 45, 256 1483 -> 79; n = 16384, k = 4096, bf16: m = 2 40 -> 26, 16 279 -> 35,
+// 256 5102 -> 368 (93 TFLOP/s).
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+struct DenseMm {
+    const void* w;  // [n, k]
+    const float* x;  // [m, k]
+    float* y;        // [m, n]
+    int64_t n;
+    int m, k;
+    int mt;          // token tiles
+};
+
+template <int WK>
+struct DenseW {
+    uint4 v;
+};
+template <>
+struct DenseW<XK_BF16> {
+    uint2 v;
+};
+
+template <int WK>
+__device__ __forceinline__ void dense_load_w(DenseW<WK>& o, __amdgpu_buffer_rsrc_t r, int voff, int soff)
+{
+    if constexpr (WK == XK_BF16) {
+        typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+        const u2 t = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+        o.v = make_uint2(t.x, t.y);
+    } else {
+        o.v = bload_s(r, voff, soff);
+    }
+}
+
+template <int WK>
+__device__ __forceinline__ float dense_w(const DenseW<WK>& o, int e)
+{
+    if constexpr (WK == XK_BF16) {
+        const uint32_t u = e < 2 ? o.v.x : o.v.y;
+        return __uint_as_float((e & 1) ? (u & 0xFFFF0000u) : (u << 16));
+    } else {
+        return __uint_as_float(e == 0 ? o.v.x : (e == 1 ? o.v.y : (e == 2 ? o.v.z : o.v.w)));
+    }
+}
+
+template <int WK, int TB, int NB>
+__global__ __launch_bounds__(512, 2) void k_dense_mm(DenseMm a)
+{
+    constexpr int WB = WK == XK_BF16 ? 2 : 4;
+    constexpr int XS = 128, WS = 32 * WB;                 // bytes of a row per wave and block
+    constexpr int XW = 16 * TB * XS, WW = 16 * NB * WS;   // one stage of a wave
+    constexpr int XC = XW / 1024, WC = WW / 1024;         // its copies
+    constexpr int kSums = 32 * 256 * 4;                   // a tile's chains, after the main loop
+    constexpr int kStage = 8 * (XW + WW) > kSums ? 8 * (XW + WW) : kSums;
+    constexpr int D = 2;
+    // an array per stage: the compiler then knows which copies a read depends on
+    __shared__ __align__(1024) uint8_t lds0[kStage];
+    __shared__ __align__(1024) uint8_t lds1[kStage];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane >> 4, r = lane & 15;
+    // consecutive workgroups (on the 8 XCDs in turn) take different weight
+    // tiles; an XCD walks the token tiles of its weight tile
+    const int b8 = (int)blockIdx.x >> 3;
+    const int64_t col0 = (int64_t)((b8 / a.mt) * 8 + (blockIdx.x & 7)) * 16 * NB;
+    const int row0 = (b8 % a.mt) * 16 * TB;
+    if (col0 >= a.n) return;  // uniform
+    const int K = a.k;
+    const int nrow = min(16 * TB, a.m - row0), ncol = (int)min((int64_t)16 * NB, a.n - col0);
+    const float* xbase = a.x + (int64_t)row0 * K;
+    const char* wbase = (const char*)a.w + col0 * K * WB;
+    // rows past the end read as zero and are not stored
+    const uint32_t xbytes = (uint32_t)nrow * K * 4, wbytes = (uint32_t)ncol * K * WB;
+
+    // copies: lane -> (row, 16-byte unit); units 0 .. half - 1 are the chains
+    // 4 wave .. 4 wave + 3, the others the chains 32 above them.  Unit u of a
+    // row sits at u ^ swizzle(row), so a quarter wave's operand reads (16 rows)
+    // cover the banks once.
+    int xo[XC], wo[WC];
+#pragma unroll
+    for (int i = 0; i < XC; ++i) {
+        const int row = 8 * i + (lane >> 3), u = (lane & 7) ^ ((row >> 1) & 7);
+        xo[i] = row * K * 4 + 64 * wave + 512 * (u >> 2) + 16 * (u & 3);
+    }
+#pragma unroll
+    for (int i = 0; i < WC; ++i) {
+        if constexpr (WK == XK_BF16) {
+            const int row = 16 * i + (lane >> 2), u = (lane & 3) ^ ((row >> 2) & 3);
+            wo[i] = row * K * 2 + 32 * wave + 256 * (u >> 1) + 16 * (u & 1);
+        } else {
+            const int row = 8 * i + (lane >> 3), u = (lane & 7) ^ ((row >> 1) & 7);
+            wo[i] = row * K * 4 + 64 * wave + 512 * (u >> 2) + 16 * (u & 3);
+        }
+    }
+    const int xrd = r * XS + ((c ^ ((r >> 1) & 7)) << 4);  // chains 4 wave + c; the others at xrd ^ 64
+    const int wrd = WK == XK_BF16 ? r * WS + (((c >> 1) ^ ((r >> 2) & 3)) << 4) + 8 * (c & 1) : xrd;
+
+    v16f acc[TB][NB][2];
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int u = 0; u < NB; ++u)
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[t][u][g][v] = 0.0f;
+
+    const int full = K >> 8;  // blocks of 256 elements
+    const auto issue = [&](int j, int d) {
+        const __amdgpu_buffer_rsrc_t xr = make_rsrc(xbase, j < full ? xbytes : 0u);
+        const __amdgpu_buffer_rsrc_t wr = make_rsrc(wbase, j < full ? wbytes : 0u);
+        uint8_t* st = (d ? lds1 : lds0) + wave * (XW + WW);
+#pragma unroll
+        for (int i = 0; i < WC; ++i) copy_to_lds(wr, st + XW + 1024 * i, wo[i] + j * 256 * WB);
+#pragma unroll
+        for (int i = 0; i < XC; ++i) copy_to_lds(xr, st + 1024 * i, xo[i] + j * 1024);
+    };
+    const auto mfma4 = [&](const uint4 (&xv)[TB], const DenseW<WK> (&wv)[NB], int g) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int t = 0; t < TB; ++t) {
+                const uint4 q = xv[t];
+                const float xe = __uint_as_float(e == 0 ? q.x : (e == 1 ? q.y : (e == 2 ? q.z : q.w)));
+#pragma unroll
+                for (int u = 0; u < NB; ++u)
+                    acc[t][u][g] =
+                        __builtin_amdgcn_mfma_f32_16x16x1f32(xe, dense_w<WK>(wv[u], e), acc[t][u][g], 0, 0, 0);
+            }
+    };
+    const auto step = [&](int d) {
+        const uint8_t* st = (d ? lds1 : lds0) + wave * (XW + WW);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            uint4 xv[TB];
+            DenseW<WK> wv[NB];
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                const uint8_t* p = st + XW + 16 * u * WS + (WK == XK_BF16 ? wrd ^ (32 * g) : wrd ^ (64 * g));
+                if constexpr (WK == XK_BF16) wv[u].v = *(const uint2*)p;
+                else wv[u].v = *(const uint4*)p;
+            }
+#pragma unroll
+            for (int t = 0; t < TB; ++t) xv[t] = *(const uint4*)(st + 16 * t * XS + (xrd ^ (64 * g)));
+            mfma4(xv, wv, g);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) issue(d, d);
+    int j = 0;
+    for (; j + D <= full; j += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            // this wave's copies of block j + d have landed (it reads no other wave's)
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm((D - 1) * (XC + WC)));
+            __asm__ volatile("" ::: "memory");
+            step(d);
+            __asm__ volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);  // every read of stage d is done (its products are issued)
+            issue(j + D + d, d);
+        }
+    }
+    wait_loads();
+    __asm__ volatile("" ::: "memory");
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (j + d < full) step(d);
+    if (K & 255) {
+        // the row's last chunks: a chain past the end takes fma(0, -0, acc) = acc
+        const __amdgpu_buffer_rsrc_t xr = make_rsrc(xbase, xbytes), wr = make_rsrc(wbase, wbytes);
+        const int rem = (K & 255) >> 2;
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const int ch = 32 * g + 4 * wave + c;
+            const bool in = ch < rem;
+            uint4 xv[TB];
+            DenseW<WK> wv[NB];
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                dense_load_w<WK>(wv[u], wr, in ? (16 * u + r) * K * WB + 4 * WB * (64 * full + ch) : kOOB, 0);
+                if (!in) {
+                    if constexpr (WK == XK_BF16) wv[u].v = make_uint2(0x80008000u, 0x80008000u);
+                    else wv[u].v = make_uint4(0x80000000u, 0x80000000u, 0x80000000u, 0x80000000u);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < TB; ++t) xv[t] = bload_s(xr, in ? (16 * t + r) * K * 4 + 16 * (64 * full + ch) : kOOB, 0);
+            mfma4(xv, wv, g);
+        }
+    }
+
+    // two tiles at a time, one in each array: [chain][16 x 16 outputs]
+#pragma unroll
+    for (int p = 0; p < TB * NB; p += 2) {
+        __syncthreads();  // the arrays are no longer read
+#pragma unroll
+        for (int i = p; i < p + 2 && i < TB * NB; ++i) {
+            float* s_c = (float*)(i & 1 ? lds1 : lds0);
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                s_c[(4 * wave + (v >> 2)) * 256 + (4 * c + (v & 3)) * 16 + r] =
+                    __fadd_rn(acc[i / NB][i % NB][0][v], acc[i / NB][i % NB][1][v]);
+        }
+        __syncthreads();
+        const int i = p + (tid >> 8), e = tid & 255;
+        if (i < TB * NB) {
+            const int row = i / NB * 16 + (e >> 4), col = i % NB * 16 + (e & 15);
+            const float* s_c = (const float*)(tid >> 8 ? lds1 : lds0) + e;
+            float z[16];
+#pragma unroll
+            for (int l = 0; l < 16; ++l) z[l] = __fadd_rn(s_c[l * 256], s_c[(l + 16) * 256]);
+#pragma unroll
+            for (int h = 8; h >= 1; h >>= 1)
+#pragma unroll
+                for (int l = 0; l < h; ++l) z[l] = __fadd_rn(z[l], z[l + h]);
+            if (row < nrow && col < ncol) a.y[(int64_t)(row0 + row) * a.n + col0 + col] = z[0];
+        }
+    }
+}
+
+template <int WK, int TB, int NB>
+static void launch_dense_mm_t(DenseMm a, hipStream_t st)
+{
+    a.mt = (a.m + 16 * TB - 1) / (16 * TB);
+    const int64_t nt = (a.n + 16 * NB - 1) / (16 * NB);
+    hipLaunchKernelGGL((k_dense_mm<WK, TB, NB>), dim3((unsigned)((nt + 7) / 8 * 8 * a.mt)), dim3(512), 0, st, a);
+}
+
+hipError_t launch_dense_mm(const void* w, int wkind, int64_t n, int64_t k, const float* x, int64_t m, float* y,
+                           hipStream_t st)
+{
+    DenseMm a{w, x, y, n, (int)m, (int)k, 0};
+    // 32 x 32 tiles (one workgroup per CU) when more than 16 tokens make enough
+    // of them, else 16 x 16 (two per CU); us with 16 x 16 / 32 x 32 tiles: k =
+    // 4096, n = 1024: m = 64 11 / 21, 128 20 / 23, 256 38 / 26; n = 5632: m = 16
+    // 25 / 25, 32 30 / 28, 128 91 / 70
+    const bool big = m > 16 && ((m + 31) / 32) * ((n + 31) / 32) >= 160;
+#define BTL_DENSE_MM(WKV)                                    \
+    if (wkind == WKV) {                                      \
+        if (big) launch_dense_mm_t<WKV, 2, 2>(a, st);        \
+        else launch_dense_mm_t<WKV, 1, 1>(a, st);            \
+        return hipGetLastError();                            \
+    }
+    BTL_DENSE_MM(XK_F32)
+    BTL_DENSE_MM(XK_BF16)
+#undef BTL_DENSE_MM
     return hipErrorInvalidValue;
 }
 

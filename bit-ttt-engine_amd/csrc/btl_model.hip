@@ -18,7 +18,8 @@
 //   k_attn_combine   merges the chunk partials of each (query, head).
 //   k_embed          token ids -> f32 rows of the embedding table.
 //   k_rmsnorm_f32    RMSNorm of f32 rows (+ a residual) into f32 rows.
-//   k_dense_gemv     a dense f32 / bf16 linear (the reference's lm_head), f32 sums.
+//   k_dense_gemv     a dense f32 / bf16 linear of one token row (the reference's
+//                    lm_head), f32 sums; more rows: k_dense_mm (btl_mm32.hip).
 //   k_greedy         argmax over the logits (last maximum wins; workgroups fold
 //                    into one device word), next id and
 //                    position bookkeeping for a device-resident decode loop.
@@ -1304,6 +1305,11 @@ hipError_t launch_dense_gemv(const void* w, int wkind, int64_t n, int64_t k, con
                              hipStream_t st)
 {
     if (n < 1 || m < 1 || m > 65535 || k < 4 || k % 4 || k > INT32_MAX / 2) return hipErrorInvalidValue;
+    // one token row: each weight is used once, streamed through registers; from
+    // two on the matrix form reads the weights once per 16 or 32 rows (n = 5632,
+    // k = 4096, f32, us: m = 1 17 / 22, 2 29 / 22)
+    if (m >= 2 && k <= kDenseMmMaxK && (n + 15) / 16 * ((m + 15) / 16) <= kDenseMmMaxTiles)
+        return launch_dense_mm(w, wkind, n, k, x, m, y, st);
     const unsigned G = (unsigned)std::min<int64_t>((n + 3) / 4, 1024);
     const dim3 grid(G, (unsigned)m), block(256);
     const bool xr = k == 4096;

@@ -865,6 +865,36 @@ def test_dense_linear(n, k, m, dt):
     assert np.abs(y.cpu().numpy() - ref).max() <= 1e-4 * max(1.0, np.abs(ref).max())
 
 
+# several token rows: the matrix form, in tiles of 16 x 16 and (from 160 of
+# them) 32 x 32 outputs; rows shorter than a block of 256 elements, a row of
+# blocks only, and last chunks that end inside a wave's and between the waves'
+# chains; ragged token and row tiles
+@pytest.mark.parametrize("n,k,m", [(33, 4, 2), (17, 252, 3), (70, 260, 17), (40, 1028, 64), (129, 768, 33),
+                                   (50, 4100, 16), (2570, 516, 40), (1030, 256, 130), (2590, 1532, 65)])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+def test_dense_linear_matrix_form(n, k, m, dt):
+    print("dense_linear matrix form", n, k, m, dt, flush=True)
+    rng = np.random.default_rng(n + k)
+    x = (rng.standard_normal((m, k)) * np.exp2(rng.integers(-20, 20, (m, k)))).astype(np.float32)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    x[0], w[0] = x[0] * 1e-36, np.abs(w[0])     # subnormal products, some rounded to -0
+    x[1, 1] = np.inf                            # only row 1 overflows or turns NaN
+    wt = torch.from_numpy(w).to(DEV)
+    wh = w
+    if dt == "bf16":
+        wt = wt.to(torch.bfloat16)
+        wh = wt.view(torch.int16).cpu().numpy().view(np.uint16)
+    xt = torch.from_numpy(x).to(DEV)
+    y = torch.full((m, n), 9.0, device=DEV)
+    code = bl.BTL_BF16 if dt == "bf16" else bl.BTL_F32
+    bl.check(bl.lib.btl_dense_linear(wt.data_ptr(), code, n, k, xt.data_ptr(), m, y.data_ptr(), stream()))
+    exp = orc.dense_linear(x, wh)
+    nan = np.isnan(exp)
+    got = y.cpu().numpy()
+    assert np.array_equal(np.isnan(got), nan) and not nan[0].any() and not np.isfinite(exp[1]).any()
+    assert np.array_equal(np.where(nan, 0, got).view(np.uint32), np.where(nan, 0, exp).view(np.uint32))
+
+
 def test_decoder_dense_head_matches_oracle():
     # the reference's dense lm_head (f32 and bf16 weights) after the ternary blocks
     cfg = TinyA()

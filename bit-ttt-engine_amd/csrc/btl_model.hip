@@ -493,8 +493,11 @@ __device__ __forceinline__ float ld_part(const float* p)
 // arithmetic: y[d] = (sum_c w_c o_c[d]) / (sum_c w_c l_c), w_c = exp(m_c -
 // max_c m_c), both sums sequential over the chunks.  part: the head's chunk
 // slots of st = hd + 2 floats.  Before the chunk count is known (cfun(): C,
-// or <= 0 for no result -> NaN), the (m, l) of the first 64 slots below cpre
-// and the values of the first 16 are loaded, all in flight together.  SC1: the
+// or <= 0 for no result -> NaN), the (m, l) of the first 128 slots below cpre
+// and the values of the first 32 are loaded, all in flight together; the values
+// of later chunks follow in two alternating blocks of 16, each loaded while the
+// other is added (read one chunk at a time, every chunk past the first 16 cost
+// a round trip to memory: one token over 6001 keys 41 us, now 24).  SC1: the
 // slots were written by other workgroups of this launch (coherent loads).
 template <bool SC1, typename CF>
 __device__ __forceinline__ void attn_merge_head(const float* part, int st, int cpre, int hd, int lane, float* y,
@@ -502,22 +505,26 @@ __device__ __forceinline__ void attn_merge_head(const float* part, int st, int c
 {
     const int d0 = lane, d1 = lane + 64;
     const bool h0 = d0 < hd, h1 = d1 < hd;
-    constexpr int kPre = 16;
+    constexpr int kB = 16;
     // every load unconditional, slots past cpre clamped to slot cpre - 1 (their
     // values are never used): a per-lane or per-slot condition here made the
     // compiler wait for the earlier loads before issuing the (m, l) loads
     const int clast = max(cpre, 1) - 1;
-    const int cl = min(lane, clast);
-    const float m_pre = ld_part<SC1>(&part[cl * st]);
-    const float l_pre = ld_part<SC1>(&part[cl * st + 1]);
-    float p0[kPre], p1[kPre];
+    const int cl = min(lane, clast), cl2 = min(lane + 64, clast);
+    const float m_pre = ld_part<SC1>(&part[cl * st]), m_pre2 = ld_part<SC1>(&part[cl2 * st]);
+    const float l_pre = ld_part<SC1>(&part[cl * st + 1]), l_pre2 = ld_part<SC1>(&part[cl2 * st + 1]);
+    float p0[2][kB], p1[2][kB];
+    const auto load = [&](int c, int i) {
 #pragma unroll
-    for (int c = 0; c < kPre; ++c) {
-        const int cc = min(c, clast);
-        p0[c] = h0 ? ld_part<SC1>(&part[cc * st + 2 + d0]) : 0.0f;
-        p1[c] = h1 ? ld_part<SC1>(&part[cc * st + 2 + d1]) : 0.0f;
-    }
-    __builtin_amdgcn_sched_barrier(0);  // all of them issue before the first use
+        for (int q = 0; q < kB; ++q) {
+            const int cc = min(c + q, clast);
+            p0[i][q] = h0 ? ld_part<SC1>(&part[cc * st + 2 + d0]) : 0.0f;
+            p1[i][q] = h1 ? ld_part<SC1>(&part[cc * st + 2 + d1]) : 0.0f;
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all of them issue before the next use
+    };
+    load(0, 0);
+    if (clast >= kB) load(kB, 1);  // uniform
     const int C = cfun();
     if (C <= 0) {
         if (h0) y[d0] = __builtin_nanf("");
@@ -527,40 +534,43 @@ __device__ __forceinline__ void attn_merge_head(const float* part, int st, int c
     float M = -__builtin_inff();
     for (int c0 = 0; c0 < C; c0 += 64) {
         const int cc = c0 + lane;
-        const float mv = c0 == 0 ? m_pre : (cc < C ? ld_part<SC1>(&part[cc * st]) : 0.0f);
+        const float mv = c0 == 0 ? m_pre : (c0 == 64 ? m_pre2 : (cc < C ? ld_part<SC1>(&part[cc * st]) : 0.0f));
         M = fmaxf(M, wave_max_f32(cc < C ? mv : -__builtin_inff()));
     }
     float L = 0.0f, O0 = 0.0f, O1 = 0.0f;
     for (int c0 = 0; c0 < C; c0 += 64) {
         const int cc = c0 + lane;
-        const float mv = c0 == 0 ? m_pre : (cc < C ? ld_part<SC1>(&part[cc * st]) : 0.0f);
-        const float lv = c0 == 0 ? l_pre : (cc < C ? ld_part<SC1>(&part[cc * st + 1]) : 0.0f);
+        float mv = m_pre, lv = l_pre;
+        if (c0 == 64) {
+            mv = m_pre2;
+            lv = l_pre2;
+        } else if (c0 > 64) {
+            mv = cc < C ? ld_part<SC1>(&part[cc * st]) : 0.0f;
+            lv = cc < C ? ld_part<SC1>(&part[cc * st + 1]) : 0.0f;
+        }
         const float w = cc < C ? btl_expf(__fsub_rn(mv, M)) : 0.0f;
         const float l = cc < C ? lv : 0.0f;
-        const int n = min(64, C - c0);
-        int u = 0;
-        if (c0 == 0) {
-#pragma unroll
-            for (int q = 0; q < kPre; ++q) {
-                if (q < n) {
-                    const float wu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), q));
-                    const float lu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l), q));
-                    L = __fadd_rn(L, __fmul_rn(wu, lu));
-                    O0 = __fadd_rn(O0, __fmul_rn(wu, p0[q]));
-                    O1 = __fadd_rn(O1, __fmul_rn(wu, p1[q]));
-                }
-            }
-            u = min(n, kPre);
-        }
-        for (; u < n; ++u) {
-            const int c = c0 + u;
+        const auto add = [&](int u, float v0, float v1) {
             const float wu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u));
             const float lu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l), u));
             L = __fadd_rn(L, __fmul_rn(wu, lu));
-            const float v0 = h0 ? ld_part<SC1>(&part[c * st + 2 + d0]) : 0.0f;
-            const float v1 = h1 ? ld_part<SC1>(&part[c * st + 2 + d1]) : 0.0f;
             O0 = __fadd_rn(O0, __fmul_rn(wu, v0));
             O1 = __fadd_rn(O1, __fmul_rn(wu, v1));
+        };
+        for (int u = 0; u < 64 && c0 + u < C; u += 2 * kB) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int ub = u + i * kB, n = C - c0 - ub;  // uniform
+                if (n >= kB) {
+#pragma unroll
+                    for (int q = 0; q < kB; ++q) add(ub + q, p0[i][q], p1[i][q]);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < kB; ++q)
+                        if (q < n) add(ub + q, p0[i][q], p1[i][q]);
+                }
+                if (n > 2 * kB) load(c0 + ub + 2 * kB, i);
+            }
         }
     }
     if (h0) y[d0] = __fdiv_rn(O0, L);

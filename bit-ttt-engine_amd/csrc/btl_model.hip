@@ -15,6 +15,8 @@
 //                    wave takes one (query, head of the GQA group) pair at a
 //                    time.  Writes the chunk's (max, sum, weighted values) per
 //                    query and head.
+//   k_attn_mm        the same partials of many queries on the f32 matrix
+//                    instructions.
 //   k_attn_combine   merges the chunk partials of each (query, head).
 //   k_embed          token ids -> f32 rows of the embedding table.
 //   k_rmsnorm_f32    RMSNorm of f32 rows (+ a residual) into f32 rows.
@@ -480,6 +482,304 @@ __global__ __launch_bounds__(1024) void k_attn_part_g(AttnArgs a)
     }
 }
 
+// btl_expf for x <= 0 or NaN, the same bits with fewer operations: no overflow
+// branch, the result scaled by one v_ldexp_f32 (rounded once, as btl_expf's two
+// exact steps round), and x below -104 taken as -104, whose result rounds to 0
+// like everything btl_expf cuts off at -103.97.
+__device__ __forceinline__ float expf_neg(float x)
+{
+    x = x < -104.0f ? -104.0f : x;
+    const float n = __builtin_rintf(__fmul_rn(x, 1.44269502162933349609375f));
+    const float r = __fsub_rn(__fsub_rn(x, __fmul_rn(n, 0.693145751953125f)),
+                              __fmul_rn(n, 1.428606765330187045037746429443359375e-6f));
+    float p = 1.98412701138295233249664306640625e-4f;
+    p = __fadd_rn(__fmul_rn(p, r), 1.3888889225199818611145019531250e-3f);
+    p = __fadd_rn(__fmul_rn(p, r), 8.3333337679505348205566406250e-3f);
+    p = __fadd_rn(__fmul_rn(p, r), 4.1666667908430099487304687500e-2f);
+    p = __fadd_rn(__fmul_rn(p, r), 0.16666667163372039794921875f);
+    p = __fadd_rn(__fmul_rn(p, r), 0.5f);
+    p = __fadd_rn(__fmul_rn(p, r), 1.0f);
+    p = __fadd_rn(__fmul_rn(p, r), 1.0f);
+    return __builtin_ldexpf(p, (int)n);
+}
+
+// ---------------------------------------------------------------------------
+// k_attn_mm: the chunk partials of many queries on the f32 matrix instructions
+// ---------------------------------------------------------------------------
+// v_mfma_f32_16x16x4_f32 adds its four products one after the other as fused
+// multiply-adds, so the chains over d of the scores and over j of the values
+// are those of attn_chunk_query, bit for bit.  A row is a (query, head of the
+// KV head's group) pair, row rho = query * rep + head; wave w of a workgroup
+// takes the 16 rows at 16 (8 blockIdx.z + w) against the 64-key chunk that the
+// workgroup dequantises into LDS.
+//   scores: A = keys (16 at a time), B = rows, so lane 16 q + r ends with the
+//     scores of row r at keys 16 t + 4 q + v (t, v < 4).  Lane 16 q + r holds
+//     q[row r][4 i + q] of every step i in registers for the whole kernel; a
+//     key row sits in LDS as [q][i], four steps per 16-byte read.
+//   softmax: the maximum and the pairwise sum of a row over its four lanes and
+//     16 registers, in attn_chunk_query's tree.
+//   values: A = rows, B = V.  The probabilities reach the A layout (lane 16 q +
+//     r: key 4 i + q) by a 4 x 4 transpose of lane quarters and registers
+//     (v_permlane32_swap, v_permlane16_swap).
+// A key that only some rows see has probability 0 for the others, and fma(0, v,
+// acc) leaves their sums as they are unless v is not finite: a workgroup whose
+// chunk holds such a value among keys past its first query sums the values in
+// plain loops that end at each row's last key.
+//
+// A workgroup keeps its rows and walks its share of their chunks: the next
+// chunk's codes are loaded during the values' products and waited for before
+// the partials' stores, which would otherwise stand in front of them in vmcnt.
+//
+// What bounds it: the f32 matrix instructions fill half of its cycles, the
+// softmax and the dequantisation about a quarter; 128 registers at four waves
+// per SIMD leave no room to run a wave's softmax beside its products.  512
+// queries over 2048 keys (32 / 8 heads of 128), us: k_attn_part_g 419 -> 170.
+constexpr int kMmRows = 128;             // rows per workgroup, 16 a wave
+constexpr int kMmVs = kAttnMaxHd + 16;  // LDS value row stride: the four keys of a step on different banks
+
+__device__ __forceinline__ void transpose4(float& a, float& b, float& c, float& d)
+{
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    const auto sw = [](float& x, float& y, auto f) {
+        const u2 t = f(__float_as_uint(x), __float_as_uint(y));
+        x = __uint_as_float(t.x);
+        y = __uint_as_float(t.y);
+    };
+    const auto s32 = [](uint32_t x, uint32_t y) { return __builtin_amdgcn_permlane32_swap(x, y, false, false); };
+    const auto s16 = [](uint32_t x, uint32_t y) { return __builtin_amdgcn_permlane16_swap(x, y, false, false); };
+    sw(a, c, s32);
+    sw(b, d, s32);
+    sw(a, b, s16);
+    sw(c, d, s16);
+}
+
+// Barrier for LDS data only: __syncthreads' release would also wait for the
+// outstanding global loads and stores.
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <int HD>
+__global__ __launch_bounds__(512, 4) void k_attn_mm(AttnArgs a, int wg_rows)
+{
+    static_assert(HD == 64 || HD == 128, "head size 64 or 128");
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    constexpr int NI = HD / 4, NE = HD / 16;
+    __shared__ __align__(16) float s_k[kAttnChunk][kAttnKs];
+    __shared__ __align__(16) float s_v[kAttnChunk][kMmVs];
+    __shared__ int s_bad;  // the last chunk with a value that is not finite at an unseen key, plus one
+    const int g = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, r = lane & 15;
+    const int rep = a.nh / a.nkv, rows = a.m * rep;
+    const int pos0 = a.d_pos ? *a.d_pos : a.pos;
+    const int row_wg = blockIdx.z * wg_rows;
+    const int first = pos0 + row_wg / rep + 1;  // keys the first row sees
+    const int t_last = min(pos0 + (min(rows, row_wg + wg_rows) - 1) / rep + 1, a.max_seq);
+    // this workgroup's share of the block's chunks (the host keeps chunks * gridDim.y below 2^32)
+    const uint32_t chunks = t_last > 0 ? (uint32_t)(t_last + kAttnChunk - 1) / kAttnChunk : 0u;
+    const int c_end = (int)(chunks * (blockIdx.y + 1u) / gridDim.y);
+    int c = (int)(chunks * blockIdx.y / gridDim.y);
+    if (c >= c_end) return;  // uniform
+
+    // this wave's rows of q (a row past the end: the last one's)
+    const int row0 = row_wg + 16 * wave;
+    const bool idle = 16 * wave >= wg_rows || row0 >= rows;  // uniform: no rows, but copies and barriers
+    const int row = min(row0 + r, rows - 1), qi = row / rep;
+    const float4* qg = (const float4*)(a.q + ((int64_t)qi * a.nh + g * rep + (row - qi * rep)) * HD);
+    // 16 elements of a key and of a value row per thread (HD == 64: half the threads)
+    const int sj = tid / NE, se = tid - sj * NE;
+    const bool stage = tid < kAttnChunk * NE;
+    uint4 kc, vc;
+    float ks, vs;
+    const auto load = [&](int ch) {
+        const int64_t rw = (int64_t)g * a.max_seq + min(ch * kAttnChunk + sj, t_last - 1);  // past the chunk: its last row
+        if (stage) {
+            kc = ((const uint4*)(a.kc + rw * HD))[se];
+            vc = ((const uint4*)(a.vc + rw * HD))[se];
+            ks = a.ksc[rw];
+            vs = a.vsc[rw];
+        }
+    };
+    load(c);
+    const int T = row0 + r < rows ? min(pos0 + qi + 1, a.max_seq) : 0;  // keys of row r
+    const int t_first = row0 + 16 <= rows ? min(pos0 + row0 / rep + 1, a.max_seq) : 0;
+    // row rw's place among the (query, head) pairs; rw / rep by a multiplication
+    // (exact for rw < 2^28)
+    const int64_t st = HD + 2, hst = a.cmax * st;
+    const uint32_t inv = rep > 1 ? (uint32_t)((0x100000000ull + rep - 1) / rep) : 0u;
+    const auto query = [&](int rw) { return rep > 1 ? (int)__umulhi((uint32_t)rw, inv) : rw; };
+    const auto pair = [&](int rw, int i) { return i * a.nh + g * rep + rw - i * rep; };
+    const int pair_r = pair(row, qi);
+    if (tid == 0) s_bad = 0;
+    lds_barrier();
+
+    for (; c < c_end; ++c) {
+        const int j0 = c * kAttnChunk;
+        // the rows of q are read again for every chunk (from L1 or L2): kept over
+        // the values' products they do not fit the 128 registers of four waves per SIMD
+        float qv[NI];
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            const float4 f = qg[4 * e + q];
+            qv[4 * e] = f.x; qv[4 * e + 1] = f.y; qv[4 * e + 2] = f.z; qv[4 * e + 3] = f.w;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // the chunk, dequantised (kv_cache.rs:122-128): kd = ((f32)code - 128) * s
+        if (stage) {
+            const uint32_t kw[4] = {kc.x, kc.y, kc.z, kc.w}, vw[4] = {vc.x, vc.y, vc.z, vc.w};
+            float kf[4][4];
+            bool bad = false;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    kf[b][w] = __fmul_rn(__fsub_rn((float)((kw[w] >> (8 * b)) & 255u), 128.0f), ks);
+                float4 vf;
+                vf.x = __fmul_rn(__fsub_rn((float)(vw[w] & 255u), 128.0f), vs);
+                vf.y = __fmul_rn(__fsub_rn((float)((vw[w] >> 8) & 255u), 128.0f), vs);
+                vf.z = __fmul_rn(__fsub_rn((float)((vw[w] >> 16) & 255u), 128.0f), vs);
+                vf.w = __fmul_rn(__fsub_rn((float)(vw[w] >> 24), 128.0f), vs);
+                // x * 0 is NaN for an infinite or NaN x
+                bad = bad || !(__fmul_rn(__fadd_rn(__fadd_rn(vf.x, vf.y), __fadd_rn(vf.z, vf.w)), 0.0f) == 0.0f);
+                *(float4*)&s_v[sj][16 * se + 4 * w] = vf;
+            }
+            // element d = 16 e + 4 w + b at [b][4 e + w]
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                *(float4*)&s_k[sj][b * NI + 4 * se] = make_float4(kf[b][0], kf[b][1], kf[b][2], kf[b][3]);
+            if (bad && j0 + sj >= first) s_bad = c + 1;
+        }
+        lds_barrier();
+        const bool plain = s_bad == c + 1;  // uniform
+        const int nj = min(kAttnChunk, T - j0);  // keys of row r here (<= 0: none)
+        const bool whole = t_first - j0 >= kAttnChunk;  // uniform: every row of the wave sees the whole chunk
+        float p[4][4];
+        if (!idle) {
+#pragma unroll
+            for (int e = 0; e < NE; ++e) transpose4(qv[4 * e], qv[4 * e + 1], qv[4 * e + 2], qv[4 * e + 3]);
+            v4f sc[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) sc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            // the four tiles interleaved, a tile's next key read right after its
+            // last product of a step, three products ahead of its use; the
+            // barriers keep the scheduler from undoing either
+            float4 kf[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) kf[t] = *(const float4*)&s_k[16 * t + r][q * NI];
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t].x, qv[4 * e], sc[t], 0, 0, 0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t].y, qv[4 * e + 1], sc[t], 0, 0, 0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t].z, qv[4 * e + 2], sc[t], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t].w, qv[4 * e + 3], sc[t], 0, 0, 0);
+                    if (e + 1 < NE) kf[t] = *(const float4*)&s_k[16 * t + r][q * NI + 4 * e + 4];
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // candle's affine(scal, 0) adds +0, which no later operation can tell
+            // from a zero of either sign
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) p[t][v] = __fmul_rn(sc[t][v], a.scal);
+            if (!whole) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) p[t][v] = 16 * t + 4 * q + v < nj ? p[t][v] : -__builtin_inff();
+            }
+            float mc = fmaxf(fmaxf(p[0][0], p[0][1]), fmaxf(p[0][2], p[0][3]));
+#pragma unroll
+            for (int t = 1; t < 4; ++t)
+                mc = fmaxf(mc, fmaxf(fmaxf(p[t][0], p[t][1]), fmaxf(p[t][2], p[t][3])));
+            mc = fmaxf(mc, __shfl_xor(mc, 16, 64));
+            mc = fmaxf(mc, __shfl_xor(mc, 32, 64));
+            float lt[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) p[t][v] = expf_neg(__fsub_rn(p[t][v], mc));  // exp(-inf) = 0: an unseen key
+                lt[t] = __fadd_rn(__fadd_rn(p[t][0], p[t][1]), __fadd_rn(p[t][2], p[t][3]));
+                lt[t] = __fadd_rn(lt[t], __shfl_xor(lt[t], 16, 64));
+                lt[t] = __fadd_rn(lt[t], __shfl_xor(lt[t], 32, 64));
+            }
+            if (q == 0 && nj > 0) {
+                float* pp = a.part + pair_r * hst + c * st;
+                pp[0] = mc;
+                pp[1] = __fadd_rn(__fadd_rn(lt[0], lt[1]), __fadd_rn(lt[2], lt[3]));
+            }
+        }
+        if (c + 1 < c_end) load(c + 1);  // lands during the values' products
+        if (plain) {
+            lds_barrier();  // every wave is done with the keys
+            static_assert(kMmRows * kAttnChunk <= kAttnChunk * kAttnKs, "the probabilities fit the keys' place");
+            float* s_p = &s_k[0][0] + wave * 16 * kAttnChunk;
+            if (!idle) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) s_p[r * kAttnChunk + 16 * t + 4 * q + v] = p[t][v];
+            }
+            lds_barrier();
+            for (int rr = 0; rr < 16 && !idle; ++rr) {
+                const int n = __shfl(nj, rr, 64);
+                if (n <= 0) continue;  // uniform
+                float* pp = a.part + __shfl(pair_r, rr, 64) * hst + c * st + 2;
+                for (int d = lane; d < HD; d += 64) {
+                    float o = 0.0f;
+                    for (int j = 0; j < n; ++j) o = __fmaf_rn(s_p[rr * kAttnChunk + j], s_v[j][d], o);
+                    pp[d] = o;
+                }
+            }
+        } else if (!idle) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) transpose4(p[t][0], p[t][1], p[t][2], p[t][3]);
+            v4f o[NE];
+#pragma unroll
+            for (int n = 0; n < NE; ++n) o[n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            float vf[2][NE];
+            const auto values = [&](int i) {
+#pragma unroll
+                for (int n = 0; n < NE; ++n) vf[i & 1][n] = s_v[4 * i + q][16 * n + r];
+            };
+            values(0);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if (i < 15) values(i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int n = 0; n < NE; ++n)
+                    o[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i >> 2][i & 3], vf[i & 1][n], o[n], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the next chunk's loads have landed by now: waited for here, not
+            // behind the stores that follow (both count in vmcnt)
+            wait_loads();
+            int rw0 = row0 + 4 * q;
+            asm volatile("" : "+v"(rw0));  // the rows' addresses formed here, not kept in registers over the loop
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int rw = rw0 + v, i = query(rw);
+                if (rw < rows && j0 < min(pos0 + i + 1, a.max_seq)) {
+                    float* pp = a.part + pair(rw, i) * hst + c * st + 2 + r;
+#pragma unroll
+                    for (int n = 0; n < NE; ++n) pp[16 * n] = o[n][v];
+                }
+            }
+        }
+        lds_barrier();  // the chunk is no longer read
+    }
+}
+
 // a partial-sum load: plain, or coherent at agent scope (sc1) when other
 // workgroups of the same launch wrote it
 template <bool SC1>
@@ -802,7 +1102,30 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t st)
         a.cmax < 1)
         return hipErrorInvalidValue;
     const dim3 grid((unsigned)a.nkv, (unsigned)a.cmax, (unsigned)((a.m + a.qb - 1) / a.qb));
-    if ((rep == 2 || rep == 4) && (a.hd == 128 || a.hd == 64) && a.qb > 1) {
+    // The matrix form from about 240000 (query, head, key) scores on; below it the
+    // 16-row tiles and their two chains of 128 products cost more than a wave per
+    // query (32 / 8 heads of 128, us with the launch and the call, before /
+    // matrix form: 32 queries over 232 keys 17 / 22, 128 over 128 25 / 25, 16
+    // over 516 23 / 17, 8 over 1544 25 / 18, 64 over 1600 113 / 43, 512 over 2048
+    // 427 / 228).  A device position is unknown here and counts as 0.
+    const int64_t pos = a.d_pos ? 0 : std::max(0, std::min(a.pos, a.max_seq));
+    const int64_t rows = (int64_t)a.m * rep;
+    if ((a.hd == 128 || a.hd == 64) && a.m > 1 && a.nh * (int64_t)a.m * (2 * pos + a.m) >= 480000 &&
+        ((uintptr_t)a.q & 15u) == 0 && rows <= 65535ll * kMmRows) {
+        const int64_t ch = a.d_pos ? a.cmax : std::min<int64_t>(a.cmax, (pos + a.m + kAttnChunk - 1) / kAttnChunk);
+        // 64 rows a workgroup (one wave with rows per SIMD) while two workgroups
+        // per CU hold the launch, then 128 rows, then several chunks a workgroup
+        // (512 over 2048: 228 us with 512 workgroups, 240 with 1024, 252 with one
+        // chunk each)
+        constexpr int64_t kResident = 512;
+        const int wg_rows = a.nkv * ((rows + 63) / 64) * ch <= kResident ? 64 : kMmRows;
+        const int64_t zb = (rows + wg_rows - 1) / wg_rows;
+        const int64_t per = std::max<int64_t>(1, (a.nkv * zb * ch + kResident - 1) / kResident);
+        const int64_t share = std::min((ch + per - 1) / per, std::min<int64_t>(65535, 0xFFFFFFFFll / (ch + 1)));
+        const dim3 gm((unsigned)a.nkv, (unsigned)share, (unsigned)zb);
+        if (a.hd == 128) hipLaunchKernelGGL(k_attn_mm<128>, gm, dim3(512), 0, st, a, wg_rows);
+        else hipLaunchKernelGGL(k_attn_mm<64>, gm, dim3(512), 0, st, a, wg_rows);
+    } else if ((rep == 2 || rep == 4) && (a.hd == 128 || a.hd == 64) && a.qb > 1) {
         // the query heads of a KV head in one wave, up to 16 queries at a time
         // (measured on MI355X, Llama-3-8B prefill of 512 tokens, us per layer:
         // 153 with one wave per head walking the block's queries one by one,

@@ -145,6 +145,40 @@ def test_attention_bitexact(nh, nkv, hd, m, pos):
         assert_same(o[i], e, "query %d" % i)
 
 
+# enough queries and keys for the matrix form: 1, 2, 3, 4 and 16 query heads per
+# KV head, both head sizes, 64 rows a workgroup and (200 queries of 32 heads)
+# 128 rows and several chunks, ragged row blocks and chunks; bad: later tokens
+# hold infinite and NaN values and keys, which earlier queries of the same
+# workgroup do not see
+@pytest.mark.parametrize("nh,nkv,hd,m,pos", [(32, 8, 128, 70, 300), (4, 2, 64, 300, 200), (3, 1, 128, 250, 500),
+                                             (16, 1, 64, 33, 900), (8, 8, 128, 130, 777), (32, 8, 128, 200, 900)])
+@pytest.mark.parametrize("bad", [False, True])
+def test_attention_matrix_form(nh, nkv, hd, m, pos, bad):
+    print("attention matrix form", nh, nkv, hd, m, pos, bad, flush=True)
+    S = pos + m + 30
+    cache = Cache(nkv, S, hd)
+    _fill_cache(cache, S, seed=nh + m + pos)
+    if bad:
+        cache.vs[0, pos + m // 2] = float("inf")
+        cache.vs[nkv - 1, pos + m - 2] = float("nan")
+        cache.ks[0, pos + m - 3] = float("nan")
+    q = np.random.default_rng(pos + 5).standard_normal((m, nh * hd)).astype(np.float32)
+    qt = torch.from_numpy(q).to(DEV)
+    kq, ks, vq, vs = cache.host()
+    rows = sorted({0, 1, m // 2 - 1, m // 2, m // 2 + 1, m - 4, m - 3, m - 2, m - 1})
+    exp = [orc.attn_decode(q[i], kq, ks, vq, vs, nh, pos + i + 1) for i in rows]
+    for d_pos in (None, torch.tensor([pos], dtype=torch.int32, device=DEV)):
+        out = torch.full((m, nh * hd), 3.0, device=DEV)
+        bl.check(bl.lib.btl_attention(qt.data_ptr(), m, nh, ctypes.byref(cache.c), 0 if d_pos is not None else pos,
+                                      d_pos.data_ptr() if d_pos is not None else None, out.data_ptr(), None, 0,
+                                      stream()))
+        o = out.cpu().numpy()
+        for i, e in zip(rows, exp):
+            nan = np.isnan(e)
+            assert np.isfinite(e).all() != (bad and i >= m // 2) and np.array_equal(np.isnan(o[i]), nan), i
+            assert_same(np.where(nan, 0, o[i]).astype(np.float32), np.where(nan, 0, e).astype(np.float32), "query %d" % i)
+
+
 def test_attention_device_position():
     nh, nkv, hd, S = 8, 2, 128, 300
     cache = Cache(nkv, S, hd)

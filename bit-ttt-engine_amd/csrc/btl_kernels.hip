@@ -2572,10 +2572,69 @@ __global__ __launch_bounds__(256) void k_quant_act(const void* x, int64_t k, int
     for (int64_t i = tid; i < k; i += 256) q[base + i] = (int8_t)quant1(load_x<XK>(x, base + i), qp.r, qp.ok);
 }
 
+// The same for k % 4 == 0 and aligned rows: four elements per load, and up to R
+// of them per thread kept between the maximum and the quantisation (k <= 1024 R);
+// R == 0 reads the row twice.  (One element per load took 5.7 us for 77 rows of
+// 3252 bf16, about one round trip to memory per 256 elements.)
+template <int XK, int R>
+__global__ __launch_bounds__(256) void k_quant_act4(const void* x, int64_t k, int8_t* q, float* s)
+{
+    __shared__ uint32_t s_w[4];
+    const int64_t row = blockIdx.x;
+    const int tid = threadIdx.x;
+    const int64_t base = row * k, nv = k >> 2;
+    const auto absmax = [](float4 v) {
+        return max(max(__float_as_uint(v.x) & 0x7FFFFFFFu, __float_as_uint(v.y) & 0x7FFFFFFFu),
+                   max(__float_as_uint(v.z) & 0x7FFFFFFFu, __float_as_uint(v.w) & 0x7FFFFFFFu));
+    };
+    typename X4<XK>::T v[R ? R : 1];
+    uint32_t amax = 0;
+    if constexpr (R > 0) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) v[i] = x4_raw<XK>(x, base + 4 * min((int64_t)tid + 256 * i, nv - 1));
+#pragma unroll
+        for (int i = 0; i < R; ++i) amax = max(amax, absmax(x4_f32<XK>(v[i])));
+    } else {
+        for (int64_t i = tid; i < nv; i += 256) amax = max(amax, absmax(x4_f32<XK>(x4_raw<XK>(x, base + 4 * i))));
+    }
+    amax = wave_max_dpp(amax);
+    if ((tid & 63) == 0) s_w[tid >> 6] = amax;
+    __syncthreads();
+    amax = max(max(s_w[0], s_w[1]), max(s_w[2], s_w[3]));
+    const QParams qp = qparams(amax);
+    if (tid == 0) s[row] = qp.s;
+    const auto put = [&](int64_t i, float4 f) {
+        const uint32_t a = (uint32_t)quant1(f.x, qp.r, qp.ok) & 255u, b = (uint32_t)quant1(f.y, qp.r, qp.ok) & 255u;
+        const uint32_t c = (uint32_t)quant1(f.z, qp.r, qp.ok) & 255u, d = (uint32_t)quant1(f.w, qp.r, qp.ok);
+        *(uint32_t*)(q + base + 4 * i) = a | (b << 8) | (c << 16) | (d << 24);
+    };
+    if constexpr (R > 0) {
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (tid + 256 * i < nv) put(tid + 256 * i, x4_f32<XK>(v[i]));
+    } else {
+        for (int64_t i = tid; i < nv; i += 256) put(i, x4_f32<XK>(x4_raw<XK>(x, base + 4 * i)));
+    }
+}
+
 hipError_t launch_quant_act(const void* x, int xkind, int64_t m, int64_t k, int8_t* q, float* s,
                             hipStream_t st)
 {
     if (m <= 0) return hipSuccess;
+    if (k >= 4 && k % 4 == 0 && ((uintptr_t)x & (xkind == XK_BF16 ? 7u : 15u)) == 0 && ((uintptr_t)q & 3u) == 0) {
+#define BTL_QA4(XKV)                                                                                          \
+    if (k <= 1024) hipLaunchKernelGGL((k_quant_act4<XKV, 1>), dim3((unsigned)m), dim3(256), 0, st, x, k, q, s); \
+    else if (k <= 4096) hipLaunchKernelGGL((k_quant_act4<XKV, 4>), dim3((unsigned)m), dim3(256), 0, st, x, k, q, s); \
+    else if (k <= 8192) hipLaunchKernelGGL((k_quant_act4<XKV, 8>), dim3((unsigned)m), dim3(256), 0, st, x, k, q, s); \
+    else hipLaunchKernelGGL((k_quant_act4<XKV, 0>), dim3((unsigned)m), dim3(256), 0, st, x, k, q, s);
+        if (xkind == XK_BF16) {
+            BTL_QA4(XK_BF16)
+        } else {
+            BTL_QA4(XK_F32)
+        }
+#undef BTL_QA4
+        return hipGetLastError();
+    }
     if (xkind == XK_BF16) hipLaunchKernelGGL(k_quant_act<XK_BF16>, dim3((unsigned)m), dim3(256), 0, st, x, k, q, s);
     else hipLaunchKernelGGL(k_quant_act<XK_F32>, dim3((unsigned)m), dim3(256), 0, st, x, k, q, s);
     return hipGetLastError();
@@ -3191,7 +3250,8 @@ hipError_t launch_ref_seq(const void* x, int xkind, int64_t m, int64_t k, const 
 }
 
 // ---------------------------------------------------------------------------
-// k_generic_i8: one wave per output, any k % 4 == 0, any alignment
+// k_generic_i8: one wave per output, any k % 4 == 0, any alignment (the sizes
+// that k_rag_i8's 32-bit offsets do not reach)
 // ---------------------------------------------------------------------------
 template <int YK>
 __global__ __launch_bounds__(256) void k_generic_i8(const int8_t* q, const float* xs, int64_t m,
@@ -3220,12 +3280,173 @@ __global__ __launch_bounds__(256) void k_generic_i8(const int8_t* q, const float
     }
 }
 
+// ---------------------------------------------------------------------------
+// k_rag_i8: any k % 4 == 0 and any alignment on the matrix cores
+// ---------------------------------------------------------------------------
+// Packed rows whose length is no multiple of 16 bytes start at any byte, so
+// they cannot be copied into LDS or loaded in aligned vectors as k_gemm_i8
+// does.  A workgroup of four waves computes a tile of 16 TB tokens x 16 NB rows,
+// wave w the 256-weight segments w, w + 4, ... of k; the waves' exact int32 sums
+// meet in LDS.  Lane 16 g + r of a segment takes the 64 weights from 64 g on of
+// weight row r and of token r, in four groups of 16, so that product j of the
+// segment has matching k on both operands: of the weights, the five dwords
+// around their 16 bytes, shifted into place by v_alignbyte (offsets from the
+// dword that holds the tile's first byte; past the dword that holds its last
+// byte the descriptor reads zeros), of the tokens, 64 bytes of the natural-order
+// int8 row, each 16 put in unpack16's order by byte permutes.  Tokens past k
+// are zeroed, which covers whatever the weight words hold there.
+//
+// What bounds it: the address unit, where a load's lanes read 16 rows.  77
+// tokens, k = 3252, n = 1001, with the quantiser and the call: 58.5 us through
+// k_generic_i8 (a wave per output), 13.2 through this, near the call's own cost.
+struct RagArgs {
+    const int8_t* q;   // [m, k]
+    const float* xs;
+    const uint8_t* w;  // [n, k / 4]
+    float sw;
+    void* y;
+    int32_t* acc_out;
+    int64_t n;
+    int m, k;
+};
+
+template <int YK, int TB, int NB>
+__global__ __launch_bounds__(256) void k_rag_i8(RagArgs a)
+{
+    __shared__ int s_acc[4][TB * NB * 256];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, r = lane & 15;
+    const int mt = (a.m + 16 * TB - 1) / (16 * TB);
+    const int64_t col0 = (int64_t)(blockIdx.x / mt) * 16 * NB;
+    const int row0 = (int)(blockIdx.x % mt) * 16 * TB;
+    const int K = a.k, rb = K >> 2;
+    const int nrow = min(16 * TB, a.m - row0), ncol = (int)min((int64_t)16 * NB, a.n - col0);
+    const int8_t* qbase = a.q + (int64_t)row0 * K;
+    const uint8_t* wfirst = a.w + col0 * rb;
+    const uint32_t skew = (uint32_t)(uintptr_t)wfirst & 3u;
+    const uint8_t* wbase = wfirst - skew;
+    // whole dwords of the tokens (k % 4 == 0; q may start at any byte) and of the weights
+    const uint32_t qskew = (uint32_t)(uintptr_t)qbase & 3u;
+    const __amdgpu_buffer_rsrc_t qr = make_rsrc(qbase - qskew, ((uint32_t)(nrow * K) + qskew + 3u) & ~3u);
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(wbase, (uint32_t)(ncol * rb + (int)skew + 3) & ~3u);
+    int qo[TB], wo[NB];
+    uint32_t ws[NB];
+#pragma unroll
+    for (int t = 0; t < TB; ++t) qo[t] = (16 * t + r) * K + 64 * g;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        const int b = (16 * u + r) * rb + 16 * g + (int)skew;
+        wo[u] = b & ~3;
+        ws[u] = (uint32_t)b & 3u;
+    }
+    v4i acc[TB][NB];
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int u = 0; u < NB; ++u) acc[t][u] = v4i{0, 0, 0, 0};
+
+    const int segs = (K + 255) >> 8;
+    for (int sg = wave; sg < segs; sg += 4) {
+        uint4 wv[NB];
+        uint32_t wl[NB];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            wv[u] = bload(wr, wo[u] + 64 * sg);
+            wl[u] = __builtin_amdgcn_raw_buffer_load_b32(wr, wo[u] + 64 * sg + 16, 0, 0);
+        }
+        uint4 qv[TB][4];
+#pragma unroll
+        for (int t = 0; t < TB; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (qskew == 0) {
+                    qv[t][j] = bload(qr, qo[t] + 256 * sg + 16 * j);
+                } else {  // uniform: tokens of a caller's buffer that is not dword aligned
+                    const int b = qo[t] + 256 * sg + 16 * j;
+                    const uint4 f = bload(qr, b);
+                    const uint32_t l = __builtin_amdgcn_raw_buffer_load_b32(qr, b + 16, 0, 0);
+                    qv[t][j] = make_uint4(__builtin_amdgcn_alignbyte(f.y, f.x, qskew), __builtin_amdgcn_alignbyte(f.z, f.y, qskew),
+                                          __builtin_amdgcn_alignbyte(f.w, f.z, qskew), __builtin_amdgcn_alignbyte(l, f.w, qskew));
+                }
+            }
+        v4i bw[NB][4];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            bw[u][0] = unpack16(__builtin_amdgcn_alignbyte(wv[u].y, wv[u].x, ws[u]));
+            bw[u][1] = unpack16(__builtin_amdgcn_alignbyte(wv[u].z, wv[u].y, ws[u]));
+            bw[u][2] = unpack16(__builtin_amdgcn_alignbyte(wv[u].w, wv[u].z, ws[u]));
+            bw[u][3] = unpack16(__builtin_amdgcn_alignbyte(wl[u], wv[u].w, ws[u]));
+        }
+        const bool tail = (sg << 8) + 256 > K;  // uniform
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int t = 0; t < TB; ++t) {
+                uint4 v = qv[t][j];
+                if (tail) {
+                    const int k0 = (sg << 8) + 64 * g + 16 * j;  // K % 4 == 0: whole words
+                    v.x = k0 < K ? v.x : 0u;
+                    v.y = k0 + 4 < K ? v.y : 0u;
+                    v.z = k0 + 8 < K ? v.z : 0u;
+                    v.w = k0 + 12 < K ? v.w : 0u;
+                }
+                const uint4 o = transpose16(v);
+                const v4i av = {(int)o.x, (int)o.y, (int)o.z, (int)o.w};
+#pragma unroll
+                for (int u = 0; u < NB; ++u)
+                    acc[t][u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bw[u][j], acc[t][u], 0, 0, 0);
+            }
+    }
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int u = 0; u < NB; ++u)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) s_acc[wave][(16 * t + 4 * g + v) * 16 * NB + 16 * u + r] = acc[t][u][v];
+    __syncthreads();
+    for (int e = tid; e < TB * NB * 256; e += 256) {
+        const int row = e / (16 * NB), col = e % (16 * NB);
+        if (row < nrow && col < ncol) {
+            const int z = s_acc[0][e] + s_acc[1][e] + s_acc[2][e] + s_acc[3][e];
+            const int64_t out = (int64_t)(row0 + row) * a.n + col0 + col;
+            store_y<YK>(a.y, out, __fmul_rn((float)z, __fmul_rn(a.xs[row0 + row], a.sw)));
+            if (a.acc_out) a.acc_out[out] = z;
+        }
+    }
+}
+
+template <int YK, int TB, int NB>
+static void launch_rag_t(const RagArgs& a, hipStream_t st)
+{
+    const int64_t tiles = ((a.m + 16 * TB - 1) / (16 * TB)) * ((a.n + 16 * NB - 1) / (16 * NB));
+    hipLaunchKernelGGL((k_rag_i8<YK, TB, NB>), dim3((unsigned)tiles), dim3(256), 0, st, a);
+}
+
 hipError_t launch_generic_i8(const int8_t* q, const float* xs, int64_t m, int64_t k,
                              const uint8_t* w, int64_t n, float sw, void* y, int ykind,
                              int32_t* acc_out, hipStream_t st)
 {
     const int64_t outs = m * n;
     if (outs <= 0) return hipSuccess;
+    // the matrix form wherever its 32-bit offsets reach (64 rows of k bytes; at
+    // most 2^24 workgroups of 256 threads)
+    if (k >= 4 && k < (1 << 24) && ((m + 15) / 16) * ((n + 15) / 16) < (1 << 24)) {
+        const RagArgs a{q, xs, w, sw, y, acc_out, n, (int)m, (int)k};
+        // 32 x 32 tiles when they fill the chip, else 16 x 16 (256 tokens, k = 4092,
+        // n = 4096: 24 / 43 us; 77, 3252, 1001: both under a launch and its call)
+        const bool big = ((m + 31) / 32) * ((n + 31) / 32) >= 256;
+#define BTL_RAG(YKV)                                  \
+    if (big) launch_rag_t<YKV, 2, 2>(a, st);          \
+    else launch_rag_t<YKV, 1, 1>(a, st);
+        if (ykind == YK_BF16) {
+            BTL_RAG(YK_BF16)
+        } else {
+            BTL_RAG(YK_F32)
+        }
+        return hipGetLastError();
+#undef BTL_RAG
+    }
     dim3 grid((unsigned)((outs + 3) / 4));
     if (ykind == YK_BF16)
         hipLaunchKernelGGL(k_generic_i8<YK_BF16>, grid, dim3(256), 0, st, q, xs, m, k, w, n, sw, y, acc_out);

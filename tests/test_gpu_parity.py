@@ -622,6 +622,33 @@ def test_large_m_sampled_rows():
     assert np.array_equal(acc.cpu().numpy()[rows], accr)
 
 
+# rows that are no multiple of 16 bytes long, weights and int8 tokens starting
+# at any byte: rows shorter than a dword and than a segment of 256 weights, a
+# last group that is full, partial and empty, tiles of 16 x 16 and (256 of
+# them) 32 x 32 outputs with ragged edges
+@pytest.mark.parametrize("m,k,n", [(1, 4, 1), (5, 4, 33), (17, 100, 70), (64, 252, 31), (2, 260, 16), (33, 3252, 129),
+                                   (515, 516, 490)])
+@pytest.mark.parametrize("off", [0, 1, 2, 3])
+def test_linear_i8_ragged_matrix_form(m, k, n, off):
+    print("i8 ragged", m, k, n, off, flush=True)
+    x = activations(m, k, seed=m + k)
+    wb = random_codes(n, k, seed=n + k, p3=0.1)
+    buf = torch.zeros(wb.size + off, dtype=torch.uint8, device=DEV)
+    buf[off:] = torch.from_numpy(wb).to(DEV)
+    pt = bl.PackedTensor(buf[off:], 0.0123, (n, k), DEV)
+    yr, q, s, accr = orc.forward_i8(x, wb, n, np.float32(0.0123))
+    acc = torch.full((m, n), 7, dtype=torch.int32, device=DEV)
+    y = bl.BitLinearHip.forward(to_dev(x, torch.float32), pt, acc_out=acc)
+    assert np.array_equal(acc.cpu().numpy(), accr)
+    assert_f32_identical(y, yr)
+    qb = torch.zeros(m * k + off, dtype=torch.int8, device=DEV)
+    qb[off:] = torch.from_numpy(np.ascontiguousarray(q)).to(DEV).reshape(-1)
+    acc.fill_(7)
+    y = bl.linear_i8(qb[off:].view(m, k), torch.from_numpy(s).to(DEV), pt, acc_out=acc)
+    assert np.array_equal(acc.cpu().numpy(), accr)
+    assert_f32_identical(y, yr)
+
+
 # --- reference fp32 semantics ---------------------------------------------------------
 
 F32_SHAPES = [(1, 2048, 5632), (3, 100, 17), (2, 36, 9), (4, 4096, 64), (1, 4, 3), (2, 8192, 8)]

@@ -60,14 +60,15 @@ __device__ __forceinline__ uint32_t wave_max_dpp(uint32_t v)
 
 // exp(x) in f32: Cody-Waite reduction x = n ln2 + r (ln2 = hi + lo, hi with 15
 // significant bits so n*hi is exact), e^r by its Taylor polynomial to r^7/7!
-// in Horner form, scaled by 2^n through exponent bits (two exact steps outside
-// the normal range).  Every step is one rounded f32 operation, so the CPU
-// oracle's restatement gives the same bits.
-__device__ __forceinline__ float btl_expf(float x)
+// in Horner form, scaled by 2^n in one rounding (v_ldexp_f32: infinity past the
+// range, subnormal results kept).  Every step is one rounded f32 operation, so
+// the CPU oracle's restatement gives the same bits; it cuts off at 88.72283936
+// and -103.97208405 where this one clamps x to 89 and -104, whose results
+// overflow and round to 0 (compared over every float on the CPU: the same).
+// A NaN passes through the comparisons.
+__device__ __forceinline__ float btl_expf_below(float x)  // x < 89 or NaN
 {
-    if (x != x) return x;
-    if (x > 88.72283935546875f) return __uint_as_float(0x7F800000u);
-    if (x < -103.97208404541016f) return 0.0f;
+    x = x < -104.0f ? -104.0f : x;
     const float n = __builtin_rintf(__fmul_rn(x, 1.44269502162933349609375f));
     const float r = __fsub_rn(__fsub_rn(x, __fmul_rn(n, 0.693145751953125f)),
                               __fmul_rn(n, 1.428606765330187045037746429443359375e-6f));
@@ -79,10 +80,12 @@ __device__ __forceinline__ float btl_expf(float x)
     p = __fadd_rn(__fmul_rn(p, r), 0.5f);
     p = __fadd_rn(__fmul_rn(p, r), 1.0f);
     p = __fadd_rn(__fmul_rn(p, r), 1.0f);
-    const int ni = (int)n;
-    if (ni > 127) return __fmul_rn(__fmul_rn(p, __uint_as_float(254u << 23)), __uint_as_float((uint32_t)(ni + 127 - 127) << 23));
-    if (ni < -126) return __fmul_rn(__fmul_rn(p, __uint_as_float((uint32_t)(ni + 64 + 127) << 23)), __uint_as_float(63u << 23));
-    return __fmul_rn(p, __uint_as_float((uint32_t)(ni + 127) << 23));
+    return __builtin_ldexpf(p, (int)n);
+}
+
+__device__ __forceinline__ float btl_expf(float x)
+{
+    return btl_expf_below(x > 89.0f ? 89.0f : x);
 }
 
 // Pairwise sum over the lanes of a wave (xor butterfly: at level j lane i adds

@@ -192,7 +192,7 @@ __device__ __forceinline__ void attn_chunk_query(const float (*s_k)[kAttnKs], co
         sc = __fadd_rn(__fmul_rn(acc, scal), 0.0f);  // candle affine(scal, 0)
     }
     const float mc = wave_max_f32(sc);
-    const float p = lane < nj ? btl_expf(__fsub_rn(sc, mc)) : 0.0f;
+    const float p = lane < nj ? btl_expf_below(__fsub_rn(sc, mc)) : 0.0f;
     const float lc = wave_pairwise_sum(p);
     sp[lane] = p;
     __syncthreads();
@@ -386,7 +386,7 @@ __device__ __forceinline__ void attn_chunk_query_g(const float (*s_k)[kAttnKs], 
 #pragma unroll
     for (int gg = 0; gg < G; ++gg) {
         mc[gg] = wave_max_f32(sc[gg]);
-        const float p = lane < nj ? btl_expf(__fsub_rn(sc[gg], mc[gg])) : 0.0f;
+        const float p = lane < nj ? btl_expf_below(__fsub_rn(sc[gg], mc[gg])) : 0.0f;
         lc[gg] = wave_pairwise_sum(p);
         sp[gg][lane] = p;
     }
@@ -480,27 +480,6 @@ __global__ __launch_bounds__(1024) void k_attn_part_g(AttnArgs a)
         attn_chunk_query_g<HD, G>(s_k, s_v, qg, &s_p[wave * G], nj, a.scal, lane, part, hstride, act);
         __syncthreads();  // s_p is rewritten by the next pass
     }
-}
-
-// btl_expf for x <= 0 or NaN, the same bits with fewer operations: no overflow
-// branch, the result scaled by one v_ldexp_f32 (rounded once, as btl_expf's two
-// exact steps round), and x below -104 taken as -104, whose result rounds to 0
-// like everything btl_expf cuts off at -103.97.
-__device__ __forceinline__ float expf_neg(float x)
-{
-    x = x < -104.0f ? -104.0f : x;
-    const float n = __builtin_rintf(__fmul_rn(x, 1.44269502162933349609375f));
-    const float r = __fsub_rn(__fsub_rn(x, __fmul_rn(n, 0.693145751953125f)),
-                              __fmul_rn(n, 1.428606765330187045037746429443359375e-6f));
-    float p = 1.98412701138295233249664306640625e-4f;
-    p = __fadd_rn(__fmul_rn(p, r), 1.3888889225199818611145019531250e-3f);
-    p = __fadd_rn(__fmul_rn(p, r), 8.3333337679505348205566406250e-3f);
-    p = __fadd_rn(__fmul_rn(p, r), 4.1666667908430099487304687500e-2f);
-    p = __fadd_rn(__fmul_rn(p, r), 0.16666667163372039794921875f);
-    p = __fadd_rn(__fmul_rn(p, r), 0.5f);
-    p = __fadd_rn(__fmul_rn(p, r), 1.0f);
-    p = __fadd_rn(__fmul_rn(p, r), 1.0f);
-    return __builtin_ldexpf(p, (int)n);
 }
 
 // ---------------------------------------------------------------------------
@@ -707,7 +686,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mm(AttnArgs a, int wg_rows)
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) p[t][v] = expf_neg(__fsub_rn(p[t][v], mc));  // exp(-inf) = 0: an unseen key
+                for (int v = 0; v < 4; ++v) p[t][v] = btl_expf_below(__fsub_rn(p[t][v], mc));  // exp(-inf) = 0: an unseen key
                 lt[t] = __fadd_rn(__fadd_rn(p[t][0], p[t][1]), __fadd_rn(p[t][2], p[t][3]));
                 lt[t] = __fadd_rn(lt[t], __shfl_xor(lt[t], 16, 64));
                 lt[t] = __fadd_rn(lt[t], __shfl_xor(lt[t], 32, 64));
@@ -848,7 +827,7 @@ __device__ __forceinline__ void attn_merge_head(const float* part, int st, int c
             mv = cc < C ? ld_part<SC1>(&part[cc * st]) : 0.0f;
             lv = cc < C ? ld_part<SC1>(&part[cc * st + 1]) : 0.0f;
         }
-        const float w = cc < C ? btl_expf(__fsub_rn(mv, M)) : 0.0f;
+        const float w = cc < C ? btl_expf_below(__fsub_rn(mv, M)) : 0.0f;
         const float l = cc < C ? lv : 0.0f;
         const auto add = [&](int u, float v0, float v1) {
             const float wu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u));

@@ -17,7 +17,8 @@
 //                    query and head.
 //   k_attn_mm        the same partials of many queries on the f32 matrix
 //                    instructions.
-//   k_attn_combine   merges the chunk partials of each (query, head).
+//   k_attn_combine   merges the chunk partials of each (query, head);
+//                    k_attn_combine1 those of one query over many workgroups.
 //   k_embed          token ids -> f32 rows of the embedding table.
 //   k_rmsnorm_f32    RMSNorm of f32 rows (+ a residual) into f32 rows.
 //   k_dense_gemv     a dense f32 / bf16 linear of one token row (the reference's
@@ -1025,6 +1026,71 @@ __global__ __launch_bounds__(64) void k_attn_combine(AttnArgs a)
     });
 }
 
+// k_attn_combine for one token: grid (nh, ceil(hd / 16)), block 256.  A workgroup
+// merges 16 dimensions of a head, so nh * hd / 16 workgroups read the partials
+// instead of one per head (or, merging in the launch, per KV head), which a
+// single CU's loads in flight held to about 15 GB/s.  Every chunk's 16 values go
+// into LDS, eight loads a thread in flight, then 16 lanes run the sums over the
+// chunks.
+constexpr int kCombineChunks = 512;  // chunks in LDS at a time
+
+__global__ __launch_bounds__(256) void k_attn_combine1(AttnArgs a)
+{
+    __shared__ float s_o[kCombineChunks][16];
+    __shared__ float s_w[kCombineChunks], s_l[kCombineChunks];
+    __shared__ float s_m[4];
+    const int h = blockIdx.x, d0 = blockIdx.y * 16;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int hd = a.hd, st = hd + 2;
+    const float* part = a.part + (int64_t)h * a.cmax * st;
+    float* y = a.out + (int64_t)h * hd;
+    const int T = (a.d_pos ? *a.d_pos : a.pos) + 1;
+    const int d = d0 + (tid & 15), dc = min(d, hd - 1);
+    if (T <= 0 || T > a.max_seq) {  // a device position outside the cache: no result
+        if (tid < 16 && d < hd) y[d] = __builtin_nanf("");
+        return;
+    }
+    const int C = (T + kAttnChunk - 1) / kAttnChunk;
+    float M = -__builtin_inff();
+    for (int c = tid; c < C; c += 256) M = fmaxf(M, part[(int64_t)c * st]);
+    M = wave_max_f32(M);
+    if (lane == 0) s_m[wave] = M;
+    __syncthreads();
+    M = fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]));
+    float L = 0.0f, O = 0.0f;
+    for (int c0 = 0; c0 < C; c0 += kCombineChunks) {
+        const int n = min(kCombineChunks, C - c0);
+        if (c0) __syncthreads();
+        for (int u = tid; u < n; u += 256) {
+            const float* p = part + (int64_t)(c0 + u) * st;
+            s_w[u] = btl_expf_below(__fsub_rn(p[0], M));
+            s_l[u] = p[1];
+        }
+        for (int u0 = tid >> 4; u0 < n; u0 += 16 * 8) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = part[(int64_t)(c0 + min(u0 + 16 * i, n - 1)) * st + 2 + dc];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (u0 + 16 * i < n) s_o[u0 + 16 * i][tid & 15] = v[i];
+        }
+        __syncthreads();
+        if (tid < 16)
+            for (int u = 0; u < n; ++u) {
+                const float w = s_w[u];
+                L = __fadd_rn(L, __fmul_rn(w, s_l[u]));
+                O = __fadd_rn(O, __fmul_rn(w, s_o[u][tid]));
+            }
+    }
+    if (tid < 16 && d < hd) y[d] = __fdiv_rn(O, L);
+}
+
+static hipError_t launch_combine1(const AttnArgs& a, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_attn_combine1, dim3((unsigned)a.nh, (unsigned)((a.hd + 15) / 16)), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_attention_dec1(const AttnArgs& a, const DecKv& kv, hipStream_t st)
 {
     const int rep = a.nh / a.nkv;
@@ -1032,7 +1098,14 @@ hipError_t launch_attention_dec1(const AttnArgs& a, const DecKv& kv, hipStream_t
         rep > kAttnMaxRep || a.cmax < 1)
         return hipErrorInvalidValue;
     const dim3 grid((unsigned)a.nkv, (unsigned)a.cmax), block((unsigned)(64 * rep));
-    if (a.ctr) {
+    // The merge in the launch is one workgroup's per KV head, so its time grows
+    // with the chunks; from 14 of them a second launch that spreads it over the
+    // chip is faster (32 / 8 heads of 128, us, in the launch / second launch: 9
+    // chunks 8.1 / 8.4, 16 8.9 / 8.3, 32 11.0 / 8.8, 94 24.0 / 15.5, 127 29.2 /
+    // 17.6).  A device position: from a cache of more than 32 chunks, where the
+    // launch costs a position below 900 up to 0.5 us.
+    const bool merge = a.ctr && (a.d_pos ? a.cmax <= 32 : a.pos < 13 * kAttnChunk);
+    if (merge) {
         if (a.nkv > kAttnMaxCtr) return hipErrorInvalidValue;
         if (a.hd == 128) hipLaunchKernelGGL((k_attn_dec1<128, true>), grid, block, 0, st, a, kv);
         else if (a.hd == 64) hipLaunchKernelGGL((k_attn_dec1<64, true>), grid, block, 0, st, a, kv);
@@ -1044,8 +1117,7 @@ hipError_t launch_attention_dec1(const AttnArgs& a, const DecKv& kv, hipStream_t
     else hipLaunchKernelGGL(k_attn_dec1<0>, grid, block, 0, st, a, kv);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_attn_combine, dim3(1u, (unsigned)a.nh), dim3(64), 0, st, a);
-    return hipGetLastError();
+    return launch_combine1(a, st);
 }
 
 // The merge counters of the one-launch decode attention: kAttnMaxCtr words per
@@ -1124,6 +1196,7 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t st)
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
+    if (a.m == 1) return launch_combine1(a, st);
     hipLaunchKernelGGL(k_attn_combine, dim3((unsigned)a.m, (unsigned)a.nh), dim3(64), 0, st, a);
     return hipGetLastError();
 }

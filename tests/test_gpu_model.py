@@ -310,6 +310,37 @@ def test_rope_append_attention_one_token_merge_sequence(nh, nkv, hd, tune):
         assert_same(out[0], orc.attn_decode(qr, kq, ks, vq, vs, nh, pos + 1), "call %d pos %d" % (i, pos))
 
 
+# the merge of many chunks in a launch of its own: the first and a later position
+# of the host's rule, a device position in a cache of more than 32 chunks, a head
+# size that is no multiple of 16 workgroup dimensions' whole blocks, and more
+# chunks than one pass of the merge holds (512)
+@pytest.mark.parametrize("nh,nkv,hd,S,pos,dpos", [(8, 2, 128, 900, 831, False), (8, 2, 128, 900, 832, False),
+                                                  (4, 4, 64, 3000, 40, True), (4, 1, 64, 3000, 2990, True),
+                                                  (2, 1, 48, 1500, 1400, False), (1, 1, 16, 33100, 33000, False)])
+def test_rope_append_attention_one_token_split_merge(nh, nkv, hd, S, pos, dpos):
+    print("rope_append_attention split merge", nh, nkv, hd, S, pos, dpos, flush=True)
+    cos, sin, dc, ds = rope_dev(500000.0, hd, S)
+    cache = Cache(nkv, S, hd)
+    _fill_cache(cache, S, seed=nh + pos)
+    rng = np.random.default_rng(pos)
+    q, k, v = (rng.standard_normal((1, n * hd)).astype(np.float32) for n in (nh, nkv, nkv))
+    qt, kt, vt = (torch.from_numpy(a).to(DEV) for a in (q, k, v))
+    d_pos = torch.tensor([pos], dtype=torch.int32, device=DEV)
+    out = torch.full((1, nh * hd), 3.0, device=DEV)
+    bl.check(bl.lib.btl_rope_append_attention(qt.data_ptr(), kt.data_ptr(), vt.data_ptr(), 1, nh, ctypes.byref(cache.c),
+                                              0 if dpos else pos, d_pos.data_ptr() if dpos else None, dc.data_ptr(),
+                                              ds.data_ptr(), out.data_ptr(), None, 0, stream()))
+    kq, ks, vq, vs = cache.host()
+    qr = orc.rope_apply(q[0].reshape(nh, hd), cos[pos], sin[pos]).reshape(-1)
+    assert_same(out[0], orc.attn_decode(qr, kq, ks, vq, vs, nh, pos + 1), "pos %d" % pos)
+    if dpos:  # a device position outside the cache: no result
+        d_pos.fill_(S)
+        bl.check(bl.lib.btl_rope_append_attention(qt.data_ptr(), kt.data_ptr(), vt.data_ptr(), 1, nh,
+                                                  ctypes.byref(cache.c), 0, d_pos.data_ptr(), dc.data_ptr(),
+                                                  ds.data_ptr(), out.data_ptr(), None, 0, stream()))
+        assert torch.isnan(out).all()
+
+
 @pytest.mark.parametrize("m,pos", [(2, 0), (17, 40), (70, 60)])
 def test_rope_append_attention_many_tokens(m, pos):
     nh, nkv, hd, S = 8, 2, 128, 200

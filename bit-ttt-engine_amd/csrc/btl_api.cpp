@@ -1320,6 +1320,30 @@ int btl_adaptive_linear(const btl_packed_t* const* bases, int nb, const void* x,
     void* wsp = nullptr;
     const hipStream_t st = (hipStream_t)stream;
     if ((rc = get_ws(dev, ws, ws_bytes, inner + (size_t)nb * ybytes, &wsp, st))) return rc;
+    const int xk = xdtype == BTL_BF16 ? btl::XK_BF16 : btl::XK_F32;
+    const int yk = ydtype == BTL_BF16 ? btl::YK_BF16 : btl::YK_F32;
+    bool fast = k >= 64 && k % 64 == 0 && k < (1 << 24) && aligned16(x);
+    for (int b = 0; b < nb; ++b) fast = fast && aligned16(bases[b]->data);
+    if (nb == 1) {  // y_0 alone: no sum
+        const Layer l{bases[0], y, nullptr};
+        return run_i8(&l, 1, x, xk, nullptr, m, k, yk, wsp, inner, st);
+    }
+    if (fast && nb <= btl::kMaxGroup && ceil_div(m, 128) * ceil_div(n, 64) >= btl::kBasesMinTiles) {
+        const WsLayout L = ws_layout(m, k, 0);
+        int8_t* q = (int8_t*)wsp + L.q_off;
+        float* s = (float*)((uint8_t*)wsp + L.s_off);
+        hipError_t e = btl::launch_quant_op(x, xk, m, k, q, s, st);
+        if (e != hipSuccess) return hip_fail(e, "quantize kernel launch");
+        const uint8_t* w[btl::kMaxGroup];
+        float sw[btl::kMaxGroup];
+        for (int b = 0; b < nb; ++b) {
+            w[b] = bases[b]->data;
+            sw[b] = bases[b]->scale;
+        }
+        e = btl::launch_gemm_i8_bases(q, s, m, k, w, sw, nb, n, y, yk, st);
+        if (e != hipSuccess) return hip_fail(e, "multi-base gemm kernel launch");
+        return BTL_OK;
+    }
     btl::AdaptiveSum sum;
     memset(&sum, 0, sizeof(sum));
     // every base's f32 output y_b = (float)acc_b * (s_x * s_b), up to kMaxGroup bases per launch
@@ -1331,15 +1355,13 @@ int btl_adaptive_linear(const btl_packed_t* const* bases, int nb, const void* x,
             ls[i] = Layer{bases[b0 + i], yb, nullptr};
             sum.ys[b0 + i] = yb;
         }
-        if ((rc = run_i8(ls, cnt, x, xdtype == BTL_BF16 ? btl::XK_BF16 : btl::XK_F32, nullptr, m, k, btl::YK_F32, wsp,
-                         inner, st)))
-            return rc;
+        if ((rc = run_i8(ls, cnt, x, xk, nullptr, m, k, btl::YK_F32, wsp, inner, st))) return rc;
     }
     // y = y_0 + y_1 + ... in base order
     sum.nb = nb;
     sum.count = m * n;
     sum.y = y;
-    sum.ykind = ydtype == BTL_BF16 ? btl::YK_BF16 : btl::YK_F32;
+    sum.ykind = yk;
     hipError_t e = btl::launch_base_sum(sum, st);
     if (e != hipSuccess) return hip_fail(e, "base sum kernel launch");
     return BTL_OK;

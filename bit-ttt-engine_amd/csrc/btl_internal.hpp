@@ -214,6 +214,14 @@ constexpr int kGemmWideMinTiles = 512;  // 256-row GEMM tiles from this many wor
 // the output has few tiles (small m); 1 when it already has kGemmSplitTarget.
 int gemm_splits(int64_t m, int64_t tiles_n, int64_t k, int* split_steps);
 hipError_t launch_gemm_i8(const GemmArgs& a, hipStream_t s);
+// the bases (2 .. kMaxGroup, equal n) of one multi-base layer, their sum in base
+// order written once; from kBasesMinTiles tiles of 128 x 64 outputs on (below
+// them the grouped launch of the bases covers the chip better: k = 4096, n =
+// 4096, three bases, us, grouped + sum / this: 256 tiles 43 / 40, with four
+// bases 47 / 51, 512 tiles 65 / 54)
+constexpr int64_t kBasesMinTiles = 400;
+hipError_t launch_gemm_i8_bases(const int8_t* q, const float* sx, int64_t m, int64_t k, const uint8_t* const* w,
+                                const float* sw, int nb, int64_t n, void* y, int ykind, hipStream_t st);
 // "k_gemm_i8<TN,WGN,NW,TM,NS>" of the calling thread's last launch_gemm_i8
 // ("" before the first)
 const char* last_gemm_form();

@@ -1729,6 +1729,178 @@ __global__ __launch_bounds__(NW * 64, 2) void k_gemm_i8(GemmArgs a)
     }
 }
 
+// ---------------------------------------------------------------------------
+// k_gemm_i8_bases: the prefill GEMM over the bases of one multi-base layer
+// ---------------------------------------------------------------------------
+// y = (float)acc_0 (s_x s_0) + (float)acc_1 (s_x s_1) + ... in base order
+// (btl_adaptive_linear) in one launch: a workgroup computes its 128 x TN output
+// tile for all NB bases, so the activations are copied and read once for NB
+// weight tiles and only y is written (through a grouped k_gemm_i8, NB f32
+// outputs were written and read back by k_base_sum).  Four waves of 128 tokens x
+// TN / 4 rows; the copies, the LDS layout and the two stages are k_gemm_i8's.
+// 512 tokens, k = 4096, n = 14336, three bases: 104 -> 86 us, 1024 tokens 192 ->
+// 148; the matrix cores and the vector ALU's unpacking take turns as in k_gemm_i8.
+struct BasesArgs {
+    const int8_t* q;  // [m, k] operand order
+    const float* sx;
+    const uint8_t* w[kMaxGroup];
+    float sw[kMaxGroup];
+    void* y;
+    int m, n, k, ykind;
+};
+
+template <int NB, int TN>
+__global__ __launch_bounds__(256, 2) void k_gemm_i8_bases(BasesArgs a)
+{
+    static_assert(TN == 128 || TN == 64, "tile of 128 or 64 output rows");
+    constexpr int TM = kGemmBM, TMB = TM / 16, TNB = TN / 64;
+    constexpr int ABytes = TM * kGemmBK, BBytes = TN * kGemmBK / 4;  // BBytes of one base
+    constexpr int Stage = ABytes + NB * BBytes;
+    constexpr int ACh = ABytes / 4096;                 // A copies (1 KB) per wave per step
+    constexpr int BCh = NB * BBytes / 1024;            // B copies of the workgroup per step
+    __shared__ __align__(1024) uint8_t lds[2 * Stage];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles_m = (a.m + TM - 1) / TM;
+    const int m0 = (blockIdx.x % tiles_m) * TM, n0 = (blockIdx.x / tiles_m) * TN;
+    const int K = a.k, N = a.n, rbs = K >> 2;
+    const int rows_a = min(TM, a.m - m0), rows_b = min(TN, N - n0);
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(a.q + (int64_t)m0 * K, (uint32_t)(rows_a * K));
+    __amdgpu_buffer_rsrc_t rb[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) rb[b] = make_rsrc(a.w[b] + (int64_t)n0 * rbs, (uint32_t)(rows_b * rbs));
+    const int steps = (K + kGemmBK - 1) / kGemmBK;
+
+    int aoff[ACh];
+#pragma unroll
+    for (int i = 0; i < ACh; ++i) {
+        const int c = wave * ACh + i;
+        const int j = c / TMB, row = (c % TMB) * 16 + (lane >> 2);
+        const int grp = (lane & 3) ^ ((row >> 1) & 3);
+        aoff[i] = row * K + j * 64 + grp * 16;
+    }
+    // B copy c of a base: 64 columns x 16 B of half c / (TN / 64)
+    constexpr int BPB = BBytes / 1024;
+    const auto issue = [&](int st, int stage) {
+        const int ko = st * kGemmBK;
+        uint8_t* base = lds + stage * Stage;
+#pragma unroll
+        for (int i = 0; i < ACh; ++i) copy_to_lds(ra, base + (wave * ACh + i) * 1024, aoff[i] + ko);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int c = 0; c < BPB; ++c)
+                if (((b * BPB + c) & 3) == wave)  // uniform
+                    copy_to_lds(rb[b], base + ABytes + b * BBytes + c * 1024,
+                                ((c % (TN / 64)) * 64 + lane) * rbs + (c / (TN / 64)) * 16 + (ko >> 2));
+    };
+    static_assert(BCh >= 1, "at least one weight copy");
+
+    v4i acc[NB][TMB][TNB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int t = 0; t < TMB; ++t)
+#pragma unroll
+            for (int c = 0; c < TNB; ++c) acc[b][t][c] = v4i{0, 0, 0, 0};
+    const int r16 = lane & 15, kq = lane >> 4;
+    const int aread = r16 * 64 + ((kq ^ ((r16 >> 1) & 3)) * 16);
+    const int bread = ABytes + (wave * TNB * 16 + r16) * 16 + kq * 4;
+    const auto compute_half = [&](const uint8_t* base, int j) {
+        v4i bop[NB][TNB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int c = 0; c < TNB; ++c)
+                bop[b][c] = unpack16(*(const uint32_t*)(base + bread + b * BBytes + j * (TN * 16) + c * 256));
+        const uint8_t* ab = base + j * (TM * 64) + aread;
+#pragma unroll
+        for (int t = 0; t < TMB; ++t) {
+            const v4i aop = *(const v4i*)(ab + t * 1024);
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int c = 0; c < TNB; ++c)
+                    acc[b][t][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(aop, bop[b][c], acc[b][t][c], 0, 0, 0);
+        }
+    };
+    issue(0, 0);
+    int st = 0;
+    for (; st + 1 < steps; ++st) {
+        const int stage = st & 1;
+        wait_loads();     // this wave's copies of step st are in LDS
+        __syncthreads();  // ... every wave's; and the other stage is no longer read
+        issue(st + 1, stage ^ 1);
+        const uint8_t* base = lds + stage * Stage;
+        compute_half(base, 0);
+        compute_half(base, 1);
+    }
+    {
+        wait_loads();
+        __syncthreads();
+        const uint8_t* base = lds + (st & 1) * Stage;
+        compute_half(base, 0);
+        if (st * kGemmBK + 64 < K) compute_half(base, 1);  // k % 128 == 64: the last step is half
+    }
+    const bool ybf = a.ykind == YK_BF16;
+    const int nb0 = n0 + wave * TNB * 16 + r16;
+#pragma unroll
+    for (int t = 0; t < TMB; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int m = m0 + t * 16 + 4 * kq + v;
+            if (m >= a.m) continue;
+            const float sx = a.sx[m];
+            float cm[NB];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) cm[b] = __fmul_rn(sx, a.sw[b]);
+#pragma unroll
+            for (int c = 0; c < TNB; ++c) {
+                const int n = nb0 + c * 16;
+                float z = __fmul_rn((float)acc[0][t][c][v], cm[0]);
+#pragma unroll
+                for (int b = 1; b < NB; ++b) z = __fadd_rn(z, __fmul_rn((float)acc[b][t][c][v], cm[b]));
+                if (n < N) {
+                    if (ybf) ((uint16_t*)a.y)[(int64_t)m * N + n] = f32_to_bf16(z);
+                    else ((float*)a.y)[(int64_t)m * N + n] = z;
+                }
+            }
+        }
+}
+
+hipError_t launch_gemm_i8_bases(const int8_t* q, const float* sx, int64_t m, int64_t k, const uint8_t* const* w,
+                                const float* sw, int nb, int64_t n, void* y, int ykind, hipStream_t st)
+{
+    if (m < 1 || n < 1 || nb < 2 || nb > kMaxGroup || k % 64 != 0 || k >= (1 << 24)) return hipErrorInvalidValue;
+    BasesArgs a{};
+    a.q = q;
+    a.sx = sx;
+    a.y = y;
+    a.m = (int)m;
+    a.n = (int)n;
+    a.k = (int)k;
+    a.ykind = ykind;
+    for (int b = 0; b < nb; ++b) {
+        a.w[b] = w[b];
+        a.sw[b] = sw[b];
+    }
+    // 64-row tiles (three workgroups per CU), or with three bases 128-row tiles (two
+    // per CU, 1.6 times as long each) where those take fewer rounds of the chip (k =
+    // 4096, n = 14336, us with 128 / 64 rows: m = 256 60 / 50, 512 86 / 91, 1024 158 /
+    // 148; two bases 55 / 40, 70 / 66, 127 / 111; four bases hold 64 rows at most)
+    const int64_t tm = (m + kGemmBM - 1) / kGemmBM;
+    const int64_t w64 = tm * ((n + 63) / 64), w128 = tm * ((n + 127) / 128);
+    const bool wide = nb == 3 && (w128 + 511) / 512 * 8 < (w64 + 767) / 768 * 5;
+#define BTL_BASES(NBV, TNV)                                                                                        \
+    if (nb == NBV && wide == (TNV == 128)) {                                                                       \
+        hipLaunchKernelGGL((k_gemm_i8_bases<NBV, TNV>), dim3((unsigned)(TNV == 128 ? w128 : w64)), dim3(256), 0, st, a); \
+        return hipGetLastError();                                                                                  \
+    }
+    BTL_BASES(2, 64) BTL_BASES(3, 64) BTL_BASES(3, 128) BTL_BASES(4, 64)
+#undef BTL_BASES
+    return hipErrorInvalidValue;
+}
+
 // k_gemm_reduce: sum the split-K partials of every output, then the epilogue
 // y = (float)acc * (s_x[m] * s_w) of its layer.  One thread per output, the
 // splits' loads issued 8 at a time.

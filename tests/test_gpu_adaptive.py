@@ -65,6 +65,27 @@ def test_adaptive_linear_bf16_and_llama_shape(m):
     assert y3.shape == (1, m, n) and torch.equal(y3.reshape(m, n), y)
 
 
+# enough 128 x 64 tiles for the launch over all bases: ragged tokens and rows, a
+# last K step that is half (k % 128 == 64), both row tiles of three bases (25001
+# rows take the 128-row one), and a count of bases past the launch's
+@pytest.mark.parametrize("m,n,k,nb", [(130, 12801, 192, 2), (130, 12801, 128, 3), (200, 25001, 64, 3), (257, 8600, 64, 4),
+                                      (130, 12801, 64, 5)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_adaptive_linear_bases_in_one_launch(m, n, k, nb, dt):
+    print("adaptive bases", m, n, k, nb, dt, flush=True)
+    rng = np.random.default_rng(m + nb)
+    packed = rng.integers(0, 256, (n, k // 4, nb), dtype=np.uint8)
+    s = (0.02 * 0.4 ** np.arange(nb)).astype(np.float32)
+    layer = bl.AdaptiveBitLinear.load(k, n, torch.from_numpy(packed).to(DEV), list(s))
+    xt = torch.from_numpy(activations(m, k, seed=m + nb)).to(DEV).to(dt)
+    y = layer.forward(xt)
+    e = orc.adaptive_forward_i8(xt.float().cpu().numpy(), packed, s, n)
+    if dt == torch.float32:
+        assert np.array_equal(y.cpu().numpy().view(np.uint32), e.view(np.uint32))
+    else:
+        assert np.array_equal(y.cpu().view(torch.int16).numpy().view(np.uint16), orc.f32_to_bf16(e))
+
+
 def test_adaptive_rejects_bad_shapes():
     packed, s = model(16, 64, 2, seed=1)
     with pytest.raises(bl.BitLinearError):

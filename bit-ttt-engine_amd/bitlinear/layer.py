@@ -2,7 +2,6 @@
 import ctypes
 import warnings
 
-import numpy as np
 import torch
 
 from ._lib import (
@@ -277,19 +276,29 @@ def ste_weight(w):
     float64 and rounded once; candle's own f32 reduction order is not vendored, so its
     last ulp is not pinned."""
     w = w.to(torch.float32)
-    s = float(np.float32(w.detach().abs().double().mean().item())) if w.numel() else float("nan")
-    inv = float(np.float32(1.0 / s)) if s != 0.0 else float("inf")
-    w_s = w * inv + 0.0
-    a = w_s.detach().abs().double()
-    w_q = (torch.sign(w_s.detach()) * torch.floor(a + 0.5).to(torch.float32)).clamp(-1.0, 1.0)
-    return (w_q - w_s).detach() + w_s
+    with torch.no_grad():
+        # the scale stays on the device: read by the host, it would make every call
+        # wait for the layer's earlier work
+        mean = torch.linalg.vector_norm(w, 1, dtype=torch.float64) / w.numel()
+        inv = mean.float().double().reciprocal().float()
+    w_s = w * inv  # the affine's + 0 only turns a -0 into +0, which (w_q - w_s) + w_s does as well
+    with torch.no_grad():
+        # round half away from zero, then clamp: 0 below one half, else the sign
+        w_q = torch.nn.functional.hardshrink(w_s, _BELOW_HALF).sign_()
+        step = w_q.sub_(w_s)
+    return step + w_s
+
+
+_BELOW_HALF = 0.5 - 2.0 ** -25  # the largest float32 below one half
 
 
 def matmul_robust(lhs, rhs):
     """TensorExt::matmul_robust (layers.rs:28-59): rhs moved to lhs's device, rank 1
     lhs as one row, rank > 2 flattened to [B*T, K] and reshaped back."""
     lhs = lhs.contiguous()
-    rhs = rhs.contiguous().to(lhs.device)
+    rhs = rhs.to(lhs.device)
+    if not (rhs.dim() == 2 and rhs.t().is_contiguous()):  # a transposed matrix is multiplied as it lies
+        rhs = rhs.contiguous()
     if lhs.dim() == 1:
         return (lhs.unsqueeze(0) @ rhs).squeeze(0)
     if lhs.dim() == 2:

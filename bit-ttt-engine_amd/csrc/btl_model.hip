@@ -1173,12 +1173,13 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t st)
         const int64_t ch = a.d_pos ? a.cmax : std::min<int64_t>(a.cmax, (pos + a.m + kAttnChunk - 1) / kAttnChunk);
         // 64 rows a workgroup (one wave with rows per SIMD) while two workgroups
         // per CU hold the launch, then 128 rows, then several chunks a workgroup
-        // (512 over 2048: 228 us with 512 workgroups, 240 with 1024, 252 with one
-        // chunk each)
+        // (512 over 2048: 222 us with 512 workgroups, 228 with 1024, 237 with one
+        // chunk each; 256 over 756, 768 workgroups: 58 with one each, 65 with two)
         constexpr int64_t kResident = 512;
         const int wg_rows = a.nkv * ((rows + 63) / 64) * ch <= kResident ? 64 : kMmRows;
         const int64_t zb = (rows + wg_rows - 1) / wg_rows;
-        const int64_t per = std::max<int64_t>(1, (a.nkv * zb * ch + kResident - 1) / kResident);
+        const int64_t wgs = a.nkv * zb * ch;
+        const int64_t per = wgs <= 800 ? 1 : (wgs + kResident - 1) / kResident;
         const int64_t share = std::min((ch + per - 1) / per, std::min<int64_t>(65535, 0xFFFFFFFFll / (ch + 1)));
         const dim3 gm((unsigned)a.nkv, (unsigned)share, (unsigned)zb);
         if (a.hd == 128) hipLaunchKernelGGL(k_attn_mm<128>, gm, dim3(512), 0, st, a, wg_rows);

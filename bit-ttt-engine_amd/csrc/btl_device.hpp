@@ -88,14 +88,27 @@ __device__ __forceinline__ float btl_expf(float x)
     return btl_expf_below(x > 89.0f ? 89.0f : x);
 }
 
-// Pairwise sum over the lanes of a wave (xor butterfly: at level j lane i adds
-// lane i ^ 2^j, which is the pairwise tree over lanes in index order -- float
-// addition commutes).  Every lane ends with the wave's sum.
+// Pairwise sum over the lanes of a wave: at level j groups of 2^j lanes are
+// added in pairs, in index order (float addition commutes, so which of a pair
+// comes first does not matter).  Every lane of a group holds its sum up to 16
+// lanes, so the mirrors within 8 and 16 lanes bring the other half's; then lane
+// 15 of a row goes to the next row and lane 31 to the upper half, and lane 63
+// has the wave's sum.  All 64 lanes call it; the result is uniform.  Six DPP
+// additions instead of six shuffles through the LDS unit, each a round trip of
+// some 120 cycles with nothing else to do (RMSNorm + QKV of one token 5.87 ->
+// 5.64 us; a 512-token prompt and 32 tokens of an 8-layer model 11.95 -> 11.84 ms).
 __device__ __forceinline__ float wave_pairwise_sum(float v)
 {
-#pragma unroll
-    for (int j = 1; j < 64; j <<= 1) v = __fadd_rn(v, __shfl_xor(v, j, 64));
-    return v;
+#define BTL_FADD_DPP(CTRL, RM) \
+    v = __fadd_rn(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, RM, 0xF, RM == 0xF)))
+    BTL_FADD_DPP(0xB1, 0xF);   // quad [1,0,3,2]
+    BTL_FADD_DPP(0x4E, 0xF);   // quad [2,3,0,1]
+    BTL_FADD_DPP(0x141, 0xF);  // row_half_mirror
+    BTL_FADD_DPP(0x140, 0xF);  // row_mirror
+    BTL_FADD_DPP(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
+    BTL_FADD_DPP(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
+#undef BTL_FADD_DPP
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
 // Correctly rounded sqrt of an f32 (the hardware v_sqrt_f32 is not): for a

@@ -714,8 +714,8 @@ def run_adaptive(gen, dev, args):
     ops = 2.0 * M * n * k * nb
     print("bench: adaptive nb=3 decode %.2f us, prefill %.1f us" % (us1, usm), file=sys.stderr, flush=True)
     return {"workload": "multi-base adaptive format, 3 bases, 4096 -> 14336 (Llama-3-8B gate), W1.58-A8, bf16 in/out; "
-                        "split once on the device, then btl_adaptive_linear (one grouped launch over the bases + "
-                        "the ordered base sum)",
+                        "split once on the device, then btl_adaptive_linear (every base's product, "
+                        "added in base order)",
             "decode_m1_us": round(us1, 2), "decode_bytes": b1, "decode_GB_s": round(b1 / us1 / 1e3, 1),
             "decode_frac_hbm": round(b1 / us1 / 1e3 / HBM_PEAK_GBS, 3),
             "prefill_m": M, "prefill_us": round(usm, 2), "prefill_TOPS": round(ops / usm / 1e6, 1),

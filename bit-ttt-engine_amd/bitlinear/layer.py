@@ -276,16 +276,15 @@ def ste_weight(w):
     float64 and rounded once; candle's own f32 reduction order is not vendored, so its
     last ulp is not pinned."""
     w = w.to(torch.float32)
-    with torch.no_grad():
-        # the scale stays on the device: read by the host, it would make every call
-        # wait for the layer's earlier work
-        mean = torch.linalg.vector_norm(w, 1, dtype=torch.float64) / w.numel()
-        inv = mean.float().double().reciprocal().float()
+    # the scale stays on the device: read by the host, it would make every call wait for
+    # the layer's earlier work.  It and the step are constants of the derivative: detached,
+    # which takes them out of forward mode as well (no_grad does not)
+    mean = torch.linalg.vector_norm(w.detach(), 1, dtype=torch.float64) / w.numel()
+    inv = mean.float().double().reciprocal().float()
     w_s = w * inv  # the affine's + 0 only turns a -0 into +0, which (w_q - w_s) + w_s does as well
-    with torch.no_grad():
-        # round half away from zero, then clamp: 0 below one half, else the sign
-        w_q = torch.nn.functional.hardshrink(w_s, _BELOW_HALF).sign_()
-        step = w_q.sub_(w_s)
+    fixed = w_s.detach()
+    # round half away from zero, then clamp: 0 below one half, else the sign
+    step = torch.nn.functional.hardshrink(fixed, _BELOW_HALF).sign_().sub_(fixed)
     return step + w_s
 
 

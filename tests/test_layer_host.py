@@ -91,6 +91,33 @@ def test_bitlinear_ste_forward_and_gradient():
     np.testing.assert_allclose(y1.detach().numpy(), ref[0], rtol=1e-5, atol=1e-5)
 
 
+# the forward-mode derivative of the training path against reverse mode: of the layer in
+# its weight and in both operands, by jvp, jacfwd and dual tensors.  f32 products of 64
+# terms and one more of n * k for the direction: 1e-4 of the largest entry covers any order
+@pytest.mark.parametrize("n,k", [(24, 64), (5, 12), (1, 4)])
+def test_bitlinear_ste_forward_mode(n, k):
+    g = torch.Generator().manual_seed(n)
+    w, x = torch.randn((n, k), generator=g) * 0.02, torch.randn((3, k), generator=g)
+    tw, tx = torch.randn((n, k), generator=g), torch.randn((3, k), generator=g)
+
+    def layer(w, x=x):
+        with warnings.catch_warnings():
+            warnings.simplefilter("ignore")
+            return bl.BitLinear.load(k, n, w, device="cpu").forward(x)
+
+    def close(a, b):
+        assert torch.count_nonzero(b) and (a - b).abs().max() <= 1e-4 * b.abs().max()
+
+    jw, jx = torch.func.jacrev(layer, (0, 1))(w, x)
+    close(torch.func.jacfwd(layer)(w), jw)
+    close(torch.func.jvp(layer, (w,), (tw,))[1], (jw * tw).sum((2, 3)))
+    close(torch.func.jvp(layer, (w, x), (tw, tx))[1], (jw * tw).sum((2, 3)) + (jx * tx).sum((2, 3)))
+    with torch.autograd.forward_ad.dual_level():
+        t = torch.autograd.forward_ad.unpack_dual(layer(torch.autograd.forward_ad.make_dual(w, tw))).tangent
+        close(t, (jw * tw).sum((2, 3)))
+    close(torch.func.jvp(ste_weight, (w,), (tw,))[1], tw * float(np_ste_weight(w.numpy())[1]))
+
+
 def test_adaptive_layer_state_and_mode_checks():
     # adaptive_linear.rs:126-127,159: no weights at all / a layer without either form
     with pytest.raises(bl.BitLinearError, match="neither legacy nor adaptive"):

@@ -262,7 +262,8 @@ class BitLinear:
                 return y.reshape(orig)
             return y
         warnings.warn("BitLinear: no packed params, using the STE training path", stacklevel=2)
-        return matmul_robust(x.to(torch.float32), ste_weight(self.weight).t())
+        # ste_weight's result is this call's own: multiplied as it lies, not copied first
+        return _matmul_rows(x.to(torch.float32).contiguous(), ste_weight(self.weight).to(x.device).t())
 
 
 def ste_weight(w):
@@ -294,10 +295,11 @@ _BELOW_HALF = 0.5 - 2.0 ** -25  # the largest float32 below one half
 def matmul_robust(lhs, rhs):
     """TensorExt::matmul_robust (layers.rs:28-59): rhs moved to lhs's device, rank 1
     lhs as one row, rank > 2 flattened to [B*T, K] and reshaped back."""
-    lhs = lhs.contiguous()
-    rhs = rhs.to(lhs.device)
-    if not (rhs.dim() == 2 and rhs.t().is_contiguous()):  # a transposed matrix is multiplied as it lies
-        rhs = rhs.contiguous()
+    return _matmul_rows(lhs.contiguous(), rhs.contiguous().to(lhs.device))
+
+
+def _matmul_rows(lhs, rhs):
+    """A contiguous lhs of any rank against the matrix rhs."""
     if lhs.dim() == 1:
         return (lhs.unsqueeze(0) @ rhs).squeeze(0)
     if lhs.dim() == 2:

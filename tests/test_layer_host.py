@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import bitlinear as bl
-from bitlinear.layer import ste_weight
+from bitlinear.layer import matmul_robust, ste_weight
 from datagen import weights
 from oracle import oracle as orc
 
@@ -116,6 +116,17 @@ def test_bitlinear_ste_forward_mode(n, k):
         t = torch.autograd.forward_ad.unpack_dual(layer(torch.autograd.forward_ad.make_dual(w, tw))).tangent
         close(t, (jw * tw).sum((2, 3)))
     close(torch.func.jvp(ste_weight, (w,), (tw,))[1], tw * float(np_ste_weight(w.numpy())[1]))
+
+
+def test_matmul_robust_keeps_its_own_transposed_operand():
+    # the gradient of lhs uses the rhs of the call, whatever its owner writes afterwards
+    g = torch.Generator().manual_seed(2)
+    w, x = torch.randn((5, 8), generator=g), torch.randn((2, 3, 8), generator=g, requires_grad=True)
+    y = matmul_robust(x, w.t())
+    exp = w.sum(0).expand(2, 3, 8).clone()
+    w.add_(1.0)
+    y.sum().backward()
+    torch.testing.assert_close(x.grad, exp, rtol=1e-6, atol=1e-6)
 
 
 def test_adaptive_layer_state_and_mode_checks():

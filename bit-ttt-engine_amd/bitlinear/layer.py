@@ -5,8 +5,8 @@ import warnings
 import torch
 
 from ._lib import (
-    BTL_ACT_F32_REF, BTL_ACT_F32_SEQ, BTL_ACT_I8, BTL_BF16, BTL_ERR_DEVICE, BTL_ERR_DTYPE, BTL_ERR_LAYOUT, BTL_F32,
-    BitLinearError, BtlPacked, check, lib,
+    BTL_ACT_F32_REF, BTL_ACT_F32_SEQ, BTL_ACT_I8, BTL_BF16, BTL_ERR_ARG, BTL_ERR_DEVICE, BTL_ERR_DTYPE, BTL_ERR_LAYOUT,
+    BTL_F32, BitLinearError, BtlPacked, check, lib,
 )
 from .packed import PackedTensor
 
@@ -276,6 +276,10 @@ def ste_weight(w):
     Gradients flow to w through w_s (d w_ste / d w = 1 / scale).  The mean is taken in
     float64 and rounded once; candle's own f32 reduction order is not vendored, so its
     last ulp is not pinned."""
+    if w.is_cuda and torch.cuda.is_current_stream_capturing():
+        # the mean's reduction clears its counters by a memory node, which replays of a
+        # graph do not run reliably
+        raise BitLinearError(BTL_ERR_ARG, "the training path cannot be captured in a graph")
     w = w.to(torch.float32)
     # the scale stays on the device: read by the host, it would make every call wait for
     # the layer's earlier work.  It and the step are constants of the derivative: detached,

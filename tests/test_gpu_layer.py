@@ -67,6 +67,21 @@ def test_bitlinear_ste_forward_and_gradient_on_gpu():
     assert yp.device.type == "cuda" and tuple(yp.shape) == (2, 5, n)
 
 
+def test_ste_training_path_refuses_capture():
+    # its mean is a library reduction that clears its counters by a memory node, which a
+    # graph must not hold: refused before anything is launched, and usable again afterwards
+    layer = bl.BitLinear(torch.from_numpy(weights(300, 512, seed=5)).to(DEV), 512, 300)
+    x = torch.ones((2, 512), device=DEV)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        y = layer.forward(x)
+        graph = torch.cuda.CUDAGraph()
+        with pytest.raises(bl.BitLinearError, match="captured"):
+            with torch.cuda.graph(graph):
+                layer.forward(x)
+        assert torch.equal(layer.forward(x), y)
+
+
 def test_matmul_robust_moves_rhs_to_the_lhs_device():
     lhs = torch.from_numpy(np.random.default_rng(3).standard_normal((3, 4, 64)).astype(np.float32)).to(DEV)
     rhs_cpu = torch.from_numpy(weights(64, 24, seed=4))

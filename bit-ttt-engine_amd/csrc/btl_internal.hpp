@@ -222,8 +222,8 @@ hipError_t launch_gemm_i8(const GemmArgs& a, hipStream_t s);
 constexpr int64_t kBasesMinTiles = 400;
 hipError_t launch_gemm_i8_bases(const int8_t* q, const float* sx, int64_t m, int64_t k, const uint8_t* const* w,
                                 const float* sw, int nb, int64_t n, void* y, int ykind, hipStream_t st);
-// "k_gemm_i8<TN,WGN,NW,TM,NS>" of the calling thread's last launch_gemm_i8
-// ("" before the first)
+// "k_gemm_i8<TN,WGN,NW,TM,NS>" or "k_gemm_i8_bases<NB,TN>" of the calling
+// thread's last launch_gemm_i8 or launch_gemm_i8_bases ("" before the first)
 const char* last_gemm_form();
 
 // Batched decode (k_gemv_bat): the GemmArgs of a GEMM with m <= 64, k % 64

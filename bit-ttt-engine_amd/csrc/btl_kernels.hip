@@ -1868,6 +1868,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_i8_bases(BasesArgs a)
         }
 }
 
+namespace {
+thread_local const char* t_gemm_form = "";
+}
+
 hipError_t launch_gemm_i8_bases(const int8_t* q, const float* sx, int64_t m, int64_t k, const uint8_t* const* w,
                                 const float* sw, int nb, int64_t n, void* y, int ykind, hipStream_t st)
 {
@@ -1893,6 +1897,7 @@ hipError_t launch_gemm_i8_bases(const int8_t* q, const float* sx, int64_t m, int
     const bool wide = nb == 3 && (w128 + 511) / 512 * 8 < (w64 + 767) / 768 * 5;
 #define BTL_BASES(NBV, TNV)                                                                                        \
     if (nb == NBV && wide == (TNV == 128)) {                                                                       \
+        t_gemm_form = "k_gemm_i8_bases<" #NBV "," #TNV ">";                                                        \
         hipLaunchKernelGGL((k_gemm_i8_bases<NBV, TNV>), dim3((unsigned)(TNV == 128 ? w128 : w64)), dim3(256), 0, st, a); \
         return hipGetLastError();                                                                                  \
     }
@@ -1958,10 +1963,6 @@ int gemm_splits(int64_t m, int64_t tiles_n, int64_t k, int* split_steps)
     const int64_t per = (steps + s - 1) / s;
     if (split_steps) *split_steps = (int)per;
     return (int)((steps + per - 1) / per);  // no empty split
-}
-
-namespace {
-thread_local const char* t_gemm_form = "";
 }
 
 const char* last_gemm_form() { return t_gemm_form; }

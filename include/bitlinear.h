@@ -139,7 +139,8 @@ int btl_check_faults(void* stream);
 
 /*
  * The instantiation ("k_gemm_i8<TN,WGN,NW,TM,NS>": output rows and waves
- * along them per tile, waves, token rows, LDS stages) of the last prefill
+ * along them per tile, waves, token rows, LDS stages; a multi-base layer's
+ * "k_gemm_i8_bases<NB,TN>": bases, output rows per tile) of the last prefill
  * GEMM this thread launched, "" before the first.  A diagnostic for tests and
  * tuning, no reference counterpart.
  */

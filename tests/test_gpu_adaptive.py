@@ -86,6 +86,14 @@ def test_adaptive_linear_bases_in_one_launch(m, n, k, nb, dt):
         assert np.array_equal(y.cpu().view(torch.int16).numpy().view(np.uint16), orc.f32_to_bf16(e))
 
 
+def test_adaptive_linear_reports_its_gemm_form():
+    for m, n, k, nb, form in [(130, 12801, 192, 3, "k_gemm_i8_bases<3,64>"), (200, 25001, 64, 3, "k_gemm_i8_bases<3,128>"),
+                              (130, 12801, 64, 5, "k_gemm_i8<"), (257, 8600, 64, 4, "k_gemm_i8_bases<4,64>")]:
+        layer = bl.AdaptiveBitLinear.load(k, n, torch.zeros((n, k // 4, nb), dtype=torch.uint8, device=DEV), [0.5] * nb)
+        layer.forward(torch.ones((m, k), device=DEV))
+        assert bl.lib.btl_last_gemm_form().decode().startswith(form), (m, n, k, nb)
+
+
 def test_adaptive_rejects_bad_shapes():
     packed, s = model(16, 64, 2, seed=1)
     with pytest.raises(bl.BitLinearError):

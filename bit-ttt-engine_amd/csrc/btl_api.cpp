@@ -1324,11 +1324,16 @@ int btl_adaptive_linear(const btl_packed_t* const* bases, int nb, const void* x,
     const int yk = ydtype == BTL_BF16 ? btl::YK_BF16 : btl::YK_F32;
     bool fast = k >= 64 && k % 64 == 0 && k < (1 << 24) && aligned16(x);
     for (int b = 0; b < nb; ++b) fast = fast && aligned16(bases[b]->data);
-    if (nb == 1) {  // y_0 alone: no sum
+    // One base: no sum, and the product writes y itself -- unless y overlaps x,
+    // which the workgroups of a decode launch read while others store.
+    const uintptr_t x0 = (uintptr_t)x, y0 = (uintptr_t)y;
+    const bool apart = x0 + (uintptr_t)(m * k) * (xdtype == BTL_BF16 ? 2 : 4) <= y0 ||
+                       y0 + (uintptr_t)(m * n) * (ydtype == BTL_BF16 ? 2 : 4) <= x0;
+    if (nb == 1 && apart) {
         const Layer l{bases[0], y, nullptr};
         return run_i8(&l, 1, x, xk, nullptr, m, k, yk, wsp, inner, st);
     }
-    if (fast && nb <= btl::kMaxGroup && ceil_div(m, 128) * ceil_div(n, 64) >= btl::kBasesMinTiles) {
+    if (fast && nb >= 2 && nb <= btl::kMaxGroup && ceil_div(m, 128) * ceil_div(n, 64) >= btl::kBasesMinTiles) {
         const WsLayout L = ws_layout(m, k, 0);
         int8_t* q = (int8_t*)wsp + L.q_off;
         float* s = (float*)((uint8_t*)wsp + L.s_off);

@@ -326,6 +326,7 @@ int btl_swiglu_linear_group(const btl_packed_t* const* w, void* const* y, int co
  *   reference counterpart): the activations quantised once per launch as
  *   btl_linear, acc_b exact per base, y = (float)acc_0 (s_x s_0) + (float)acc_1
  *   (s_x s_1) + ... in base order.  bases: nb btl_packed_t of equal shape.
+ *   y may overlap x.
  *   ws: btl_adaptive_workspace_bytes (or NULL: the library's).
  */
 int btl_adaptive_split(const uint8_t* packed, int64_t n, int64_t k, int nb, uint8_t* const* out, void* stream);

@@ -86,6 +86,29 @@ def test_adaptive_linear_bases_in_one_launch(m, n, k, nb, dt):
         assert np.array_equal(y.cpu().view(torch.int16).numpy().view(np.uint16), orc.f32_to_bf16(e))
 
 
+# y over x (the whole buffer, or from its second row on): x is read before y is written on
+# every route, also with one base, whose product otherwise writes y itself
+@pytest.mark.parametrize("m", [1, 2, 7, 33, 130])
+@pytest.mark.parametrize("nb,n,k", [(1, 1024, 1024), (3, 1024, 1024), (1, 2048, 1024), (1, 12864, 64), (3, 25728, 64)])
+def test_adaptive_linear_output_over_its_input(m, nb, n, k):
+    print("adaptive in place", m, nb, n, k, flush=True)
+    rng = np.random.default_rng(m + nb + n)
+    packed = rng.integers(0, 256, (n, k // 4, nb), dtype=np.uint8)
+    s = (0.02 * 0.4 ** np.arange(nb)).astype(np.float32)
+    bases = bl.split_bases(torch.from_numpy(packed).to(DEV), n, k, list(s))
+    cs = [b.as_c() for b in bases]
+    arr = (ctypes.POINTER(bl.BtlPacked) * nb)(*[ctypes.pointer(c) for c in cs])
+    x = activations(m, k, seed=m)
+    e = orc.adaptive_forward_i8(x, packed, s, n)
+    for row in (0, 1):
+        buf = torch.zeros((m * max(n, k) + k,), device=DEV)
+        buf[:m * k] = torch.from_numpy(x).to(DEV).reshape(-1)
+        y = buf[row * k:row * k + m * n]
+        bl.check(bl.lib.btl_adaptive_linear(arr, nb, buf.data_ptr(), bl.BTL_F32, m, k, y.data_ptr(), bl.BTL_F32, None, 0,
+                                            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        assert np.array_equal(y.cpu().numpy().reshape(m, n).view(np.uint32), e.view(np.uint32)), row
+
+
 def test_adaptive_linear_reports_its_gemm_form():
     for m, n, k, nb, form in [(130, 12801, 192, 3, "k_gemm_i8_bases<3,64>"), (200, 25001, 64, 3, "k_gemm_i8_bases<3,128>"),
                               (130, 12801, 64, 5, "k_gemm_i8<"), (257, 8600, 64, 4, "k_gemm_i8_bases<4,64>")]:

@@ -1333,7 +1333,7 @@ int btl_adaptive_linear(const btl_packed_t* const* bases, int nb, const void* x,
         const Layer l{bases[0], y, nullptr};
         return run_i8(&l, 1, x, xk, nullptr, m, k, yk, wsp, inner, st);
     }
-    if (fast && nb >= 2 && nb <= btl::kMaxGroup && ceil_div(m, 128) * ceil_div(n, 64) >= btl::kBasesMinTiles) {
+    if (fast && btl::bases_in_one_launch(m, n, k, nb)) {
         const WsLayout L = ws_layout(m, k, 0);
         int8_t* q = (int8_t*)wsp + L.q_off;
         float* s = (float*)((uint8_t*)wsp + L.s_off);

@@ -215,11 +215,23 @@ constexpr int kGemmWideMinTiles = 512;  // 256-row GEMM tiles from this many wor
 int gemm_splits(int64_t m, int64_t tiles_n, int64_t k, int* split_steps);
 hipError_t launch_gemm_i8(const GemmArgs& a, hipStream_t s);
 // the bases (2 .. kMaxGroup, equal n) of one multi-base layer, their sum in base
-// order written once; from kBasesMinTiles tiles of 128 x 64 outputs on (below
-// them the grouped launch of the bases covers the chip better: k = 4096, n =
-// 4096, three bases, us, grouped + sum / this: 256 tiles 43 / 40, with four
-// bases 47 / 51, 512 tiles 65 / 54)
-constexpr int64_t kBasesMinTiles = 400;
+// order written once.  Through the grouped launch of the bases and their sum
+// instead (us, grouped / one launch):
+//   below 400 tiles of 128 x 64 outputs, where that covers the chip better (k =
+//     4096, n = 4096, three bases: 256 tiles 43 / 40, with four bases 47 / 51,
+//     512 tiles 65 / 54);
+//   up to 64 tokens, most of a 128-token tile being padding, where the layer is
+//     wide enough for the tiles (n > 25536): k = 4096, n = 28672, three bases,
+//     m = 1 18.8 / 38.2, 16 30.8 / 39.8, 64 41.9 / 42.7, 65 52.3 / 42.7.  The
+//     decode routes lose on a short K, so from 3 tokens on up to k = 1024 (m = 16,
+//     n = 25600: 23.6 / 14.2), and from 17 tokens on with at most three bases up
+//     to k = 3072 (m = 20 and 32, n = 28672 and 51200: 0 to -29 %; four bases
+//     -26 to +7 %).
+inline bool bases_in_one_launch(int64_t m, int64_t n, int64_t k, int nb)
+{
+    if (nb < 2 || nb > kMaxGroup || (m + 127) / 128 * ((n + 63) / 64) < 400) return false;
+    return m > 64 || (m >= 3 && k <= 1024) || (m > 16 && nb <= 3 && k <= 3072);
+}
 hipError_t launch_gemm_i8_bases(const int8_t* q, const float* sx, int64_t m, int64_t k, const uint8_t* const* w,
                                 const float* sw, int nb, int64_t n, void* y, int ykind, hipStream_t st);
 // "k_gemm_i8<TN,WGN,NW,TM,NS>" or "k_gemm_i8_bases<NB,TN>" of the calling

@@ -9,6 +9,7 @@ import torch
 
 import bitlinear as bl
 from datagen import activations, pack_interleaved_2bit, rvq_bases, weights
+from launches import launched
 from oracle import oracle as orc
 
 pytestmark = [pytest.mark.gpu,
@@ -107,6 +108,26 @@ def test_adaptive_linear_output_over_its_input(m, nb, n, k):
         bl.check(bl.lib.btl_adaptive_linear(arr, nb, buf.data_ptr(), bl.BTL_F32, m, k, y.data_ptr(), bl.BTL_F32, None, 0,
                                             ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
         assert np.array_equal(y.cpu().numpy().reshape(m, n).view(np.uint32), e.view(np.uint32)), row
+
+
+# layers wide enough for the one launch at every token count: few tokens keep the grouped
+# launch where its tiles would be padding.  Columns checked: the first and last 200
+@pytest.mark.parametrize("m,k,nb,one", [(1, 64, 3, False), (2, 1024, 2, False), (3, 1024, 2, True), (4, 1088, 3, False),
+                                        (16, 1088, 3, False), (17, 1088, 3, True), (17, 1088, 4, False),
+                                        (32, 3136, 2, False), (64, 1088, 4, False), (65, 1088, 4, True)])
+def test_adaptive_linear_few_tokens_of_a_wide_layer(m, k, nb, one):
+    print("adaptive few tokens", m, k, nb, flush=True)
+    n = 25601
+    rng = np.random.default_rng(m + k)
+    packed = rng.integers(0, 256, (n, k // 4, nb), dtype=np.uint8)
+    s = (0.02 * 0.4 ** np.arange(nb)).astype(np.float32)
+    layer = bl.AdaptiveBitLinear.load(k, n, torch.from_numpy(packed).to(DEV), list(s))
+    xt = torch.from_numpy(activations(m, k, seed=m)).to(DEV)
+    y = layer.forward(xt).cpu().numpy()
+    cols = np.r_[:200, n - 200:n]
+    e = orc.adaptive_forward_i8(xt.cpu().numpy(), packed[cols], s, cols.size)
+    assert np.array_equal(y[:, cols].view(np.uint32), e.view(np.uint32))
+    assert any("k_gemm_i8_bases" in f for f in launched(lambda: layer.forward(xt))) == one
 
 
 def test_adaptive_linear_reports_its_gemm_form():

@@ -201,6 +201,7 @@ class BitLlamaHip:
         self._ws_n = need
         self.pos = 0
         self.graph = None
+        self._graph_until = 0  # the position from which decode_steps captures anew
 
     # ------------------------------------------------------------------ steps
     def _stream(self):
@@ -208,8 +209,8 @@ class BitLlamaHip:
 
     def _run(self, m, pos, d_pos, ids):
         """One forward of m rows, token ids in the device int32 tensor `ids`, at
-        positions pos.. (or *d_pos.. when d_pos is a device tensor); leaves the last
-        row's logits in self.logits."""
+        positions pos.. (or *d_pos.. when d_pos is a device tensor, pos then the host's
+        estimate of it); leaves the last row's logits in self.logits."""
         c, st = self.cfg, self._stream()
         ws, wn = self._ws, self._ws_n
         dp = ctypes.c_void_p(d_pos.data_ptr()) if d_pos is not None else None
@@ -384,7 +385,7 @@ class BitLlamaHip:
         """One decode step with the position on the device: the token in next_id at
         position *d_pos through the blocks and the head, then the greedy pick
         (next_id, log[*d_pos + 1], ++*d_pos)."""
-        self._run(1, 0, self.d_pos, self.next_id)
+        self._run(1, self.pos, self.d_pos, self.next_id)
         check(lib.btl_greedy_next(self.logits.data_ptr(), self.cfg.vocab, self.next_id.data_ptr(),
                                   self.d_pos.data_ptr(), self.log.data_ptr(), self.log.numel(), self._stream()))
 
@@ -400,6 +401,7 @@ class BitLlamaHip:
                 self._step_device()
         torch.cuda.synchronize(self.dev)
         self.graph = g
+        self._graph_until = max(1024, 2 * self.pos)
         return g
 
     def start_decode(self):
@@ -409,17 +411,21 @@ class BitLlamaHip:
             self.log[self.pos:self.pos + 1].copy_(self.next_id)
 
     def decode_steps(self, n, use_graph=True):
-        """n greedy steps on the device, no host synchronisation in between; the
-        tokens accumulate in self.log."""
+        """n greedy steps on the device; the tokens accumulate in self.log.  No host
+        synchronisation in between, but for a new capture of the step when the
+        position has doubled since the last one, and is 1024 at least: the launches
+        of the attention are chosen by it."""
         if self.pos + n > self.cfg.max_seq:
             raise ValueError("%d steps from position %d overflow the cache of %d rows"
                              % (n, self.pos, self.cfg.max_seq))
         for _ in range(n):
             if use_graph and self.graph is not None:
+                if self.pos >= self._graph_until:
+                    self.capture_decode()
                 self.graph.replay()
             else:
                 self._step_device()
-        self.pos += n
+            self.pos += 1
 
     def generate(self, prompt_ids, max_tokens, use_graph=True):
         """Llama::stream_completion at temperature 0 (llama.rs:471-530): prefill, then

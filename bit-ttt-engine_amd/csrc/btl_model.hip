@@ -1098,6 +1098,22 @@ static hipError_t launch_combine1(const AttnArgs& a, hipStream_t st)
     return hipGetLastError();
 }
 
+// Whether one token's chunks are merged in the launch (one workgroup per KV head, so
+// its time grows with the chunks) or by a second launch spread over the chip, which
+// has to wait until the launch's workgroups past the position have come and gone.
+// 32 / 8 heads of 128, us, in the launch / second launch: cache of 128 chunks (1024
+// workgroups), 9 chunks in use 8.0 / 8.2, 13 8.5 / 8.5, 16 8.8 / 8.4, 32 10.9 / 8.9,
+// 94 23.6 / 15.1; of 512 (4096) 16 11.9 / 14.5, 48 17.2 / 17.3, 94 26.4 / 20.9;
+// 32 / 32 heads in a cache of 512 (16384) 48 61.3 / 62.5, 94 75.8 / 75.6.  Small
+// heads of a large group are merged faster: 32 / 4 of 64, 512 workgroups, 16 chunks
+// 7.5 / 7.6, 17 7.9 / 7.8.  With a device position a.pos is the caller's estimate.
+static bool dec1_merges(const AttnArgs& a, int rep)
+{
+    const int64_t wgs = (int64_t)a.nkv * a.cmax;
+    const int64_t most = (rep >= 4 && a.hd <= 64 ? 17 : 13) + std::min<int64_t>(std::max<int64_t>(wgs - 1024, 0) / 80, 48);
+    return a.pos / kAttnChunk < most;
+}
+
 hipError_t launch_attention_dec1(const AttnArgs& a, const DecKv& kv, hipStream_t st)
 {
     const int rep = a.nh / a.nkv;
@@ -1105,13 +1121,7 @@ hipError_t launch_attention_dec1(const AttnArgs& a, const DecKv& kv, hipStream_t
         rep > kAttnMaxRep || a.cmax < 1)
         return hipErrorInvalidValue;
     const dim3 grid((unsigned)a.nkv, (unsigned)a.cmax), block((unsigned)(64 * rep));
-    // The merge in the launch is one workgroup's per KV head, so its time grows
-    // with the chunks; from 14 of them a second launch that spreads it over the
-    // chip is faster (32 / 8 heads of 128, us, in the launch / second launch: 9
-    // chunks 8.1 / 8.4, 16 8.9 / 8.3, 32 11.0 / 8.8, 94 24.0 / 15.5, 127 29.2 /
-    // 17.6).  A device position: from a cache of more than 32 chunks, where the
-    // launch costs a position below 900 up to 0.5 us.
-    const bool merge = a.ctr && (a.d_pos ? a.cmax <= 32 : a.pos < 13 * kAttnChunk);
+    const bool merge = a.ctr && dec1_merges(a, rep);
     if (merge) {
         if (a.nkv > kAttnMaxCtr) return hipErrorInvalidValue;
         if (a.hd == 128) hipLaunchKernelGGL((k_attn_dec1<128, true>), grid, block, 0, st, a, kv);

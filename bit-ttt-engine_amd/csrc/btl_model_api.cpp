@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <vector>
@@ -48,6 +49,9 @@ int check_cache(const btl_kv_q8_t* c, int64_t n_heads)
         return fail_msg(BTL_ERR_SHAPE, "KV cache too large");
     return BTL_OK;
 }
+
+// the position, or with a device position the caller's estimate of it (any value)
+int host_pos(int64_t pos, const btl_kv_q8_t* c) { return (int)std::min(std::max(pos, (int64_t)0), c->max_seq - 1); }
 
 int check_pos(int64_t pos, int64_t m, const int32_t* d_pos, const btl_kv_q8_t* c)
 {
@@ -160,7 +164,7 @@ int btl_attention(const float* q, int64_t m, int64_t n_heads, const btl_kv_q8_t*
     a.ksc = cache->k_scale;
     a.vsc = cache->v_scale;
     a.d_pos = d_pos;
-    a.pos = (int)pos;
+    a.pos = host_pos(pos, cache);
     a.m = (int)m;
     a.nh = (int)n_heads;
     a.nkv = (int)cache->n_kv_heads;
@@ -199,7 +203,7 @@ int btl_rope_append_attention(const float* q, const float* k, const float* v, in
     a.ksc = cache->k_scale;
     a.vsc = cache->v_scale;
     a.d_pos = d_pos;
-    a.pos = (int)pos;
+    a.pos = host_pos(pos, cache);
     a.m = (int)m;
     a.nh = (int)n_heads;
     a.nkv = (int)cache->n_kv_heads;

@@ -102,11 +102,14 @@ int btl_attention(const float* q, int64_t m, int64_t n_heads, const btl_kv_q8_t*
  * k and v, attention -- btl_rope_kv_append then btl_attention, same results
  * bit for bit.  q [m, n_heads * head_dim], k, v [m, n_kv * head_dim] raw
  * projection outputs (not modified), out [m, n_heads * head_dim].  For one
- * token (m == 1, head_dim % 16 == 0) the RoPE, the append, the attention and
- * the merge of its key chunks run in one launch (n_kv <= 64; the last
- * workgroup of a KV head merges, counted on per-device counters that every
- * launch leaves at zero, so such calls on one device must not overlap in
- * time -- order them on one stream, as the workspace already asks).
+ * token (m == 1, head_dim % 16 == 0) the RoPE, the append and the attention
+ * run in one launch, and up to some 13 key chunks (more in a long cache) their
+ * merge as well (n_kv <= 64; the last workgroup of a KV head merges, counted on
+ * per-device counters that every launch leaves at zero, so such calls on one
+ * device must not overlap in time -- order them on one stream, as the workspace
+ * already asks); past that a second launch merges.  With d_pos, pos is the
+ * caller's estimate of *d_pos and chooses between the two only: any value gives
+ * the same results, 0 the merge in the launch.
  * ws: btl_attention_workspace_bytes (it covers the rotated queries too).  A
  * device position outside the cache gives NaN outputs and no append.
  */

@@ -13,6 +13,7 @@ import torch
 
 import bitlinear as bl
 from bitlinear.model import BitLlamaHip
+from launches import launched
 from oracle import oracle as orc
 from oracle.llama_oracle import OracleLlama
 from test_model_oracle import TinyCfg, tiny_weights
@@ -339,6 +340,41 @@ def test_rope_append_attention_one_token_split_merge(nh, nkv, hd, S, pos, dpos):
                                                   ctypes.byref(cache.c), 0, d_pos.data_ptr(), dc.data_ptr(),
                                                   ds.data_ptr(), out.data_ptr(), None, 0, stream()))
         assert torch.isnan(out).all()
+
+
+# one launch or two, by the position and the cache's workgroups: what the launches are,
+# and the same results whatever estimate a call with a device position gives
+@pytest.mark.parametrize("nh,nkv,hd,S,pos,one", [(8, 2, 128, 900, 831, True), (8, 2, 128, 900, 832, False),
+                                                 (8, 8, 128, 9000, 40, True), (32, 4, 64, 2100, 1087, True),
+                                                 (32, 4, 64, 2100, 1088, False), (8, 8, 128, 32768, 3263, True),
+                                                 (8, 8, 128, 32768, 3264, False)])
+def test_rope_append_attention_one_token_launches(nh, nkv, hd, S, pos, one):
+    print("rope_append_attention launches", nh, nkv, hd, S, pos, flush=True)
+    cos, sin, dc, ds = rope_dev(500000.0, hd, pos + 1)
+    dc, ds = (torch.cat((t, t.new_zeros((S - pos - 1, hd // 2)))) for t in (dc, ds))
+    cache = Cache(nkv, S, hd)
+    _fill_cache(cache, S, seed=nh + pos)
+    rng = np.random.default_rng(pos)
+    q, k, v = (rng.standard_normal((1, n * hd)).astype(np.float32) for n in (nh, nkv, nkv))
+    qt, kt, vt = (torch.from_numpy(a).to(DEV) for a in (q, k, v))
+    d_pos = torch.tensor([pos], dtype=torch.int32, device=DEV)
+    out = torch.empty((1, nh * hd), device=DEV)
+
+    def call(host, dev):
+        bl.check(bl.lib.btl_rope_append_attention(qt.data_ptr(), kt.data_ptr(), vt.data_ptr(), 1, nh,
+                                                  ctypes.byref(cache.c), host, d_pos.data_ptr() if dev else None,
+                                                  dc.data_ptr(), ds.data_ptr(), out.data_ptr(), None, 0, stream()))
+
+    exp = None
+    for host, dev, single in ((pos, False, one), (pos, True, one), (0, True, True), (-1 << 40, True, True),
+                              (1 << 40, True, S // 64 < 14)):
+        out.fill_(3.0)
+        call(host, dev)
+        if exp is None:
+            qr = orc.rope_apply(q[0].reshape(nh, hd), cos[pos], sin[pos]).reshape(-1)
+            exp = orc.attn_decode(qr, *cache.host(), nh, pos + 1)
+        assert_same(out[0], exp, "estimate %d" % host)
+        assert len(launched(lambda: call(host, dev))) == (1 if single else 2), (host, dev)
 
 
 @pytest.mark.parametrize("m,pos", [(2, 0), (17, 40), (70, 60)])
@@ -704,6 +740,29 @@ def test_decoder_prefill_equals_token_by_token(cfg_cls):
     for li in range(cfg.n_layers):
         assert torch.equal(a.caches[li].k, b.caches[li].k) and torch.equal(a.caches[li].v, b.caches[li].v)
         assert torch.equal(a.caches[li].k_scale, b.caches[li].k_scale)
+
+
+def test_decoder_steps_over_a_new_capture():
+    # the step is captured anew at position 1024 (then where the position has doubled)
+    cfg = TinyA()
+    cfg.max_seq = 2300
+    w = tiny_weights(cfg, seed=5)
+    prompt = np.random.default_rng(3).integers(0, cfg.vocab, 505)
+    logs = []
+    for use_graph in (True, False):
+        gm = gpu_model(cfg, w)
+        gm.prefill(prompt)
+        gm.greedy()
+        gm.start_decode()
+        if use_graph:
+            first = gm.capture_decode()
+            for n in (519, 1, 30):
+                gm.decode_steps(n)
+                assert (gm.graph is first) == (gm.pos <= 1024) and gm.d_pos.item() == gm.pos
+        else:
+            gm.decode_steps(550, use_graph=False)
+        logs.append(gm.log[505:1056].clone())
+    assert gm.pos == 1055 and torch.equal(*logs)
 
 
 @pytest.mark.parametrize("use_graph", [False, True])

@@ -1175,10 +1175,18 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t st)
     // query (32 / 8 heads of 128, us with the launch and the call, before /
     // matrix form: 32 queries over 232 keys 17 / 22, 128 over 128 25 / 25, 16
     // over 516 23 / 17, 8 over 1544 25 / 18, 64 over 1600 113 / 43, 512 over 2048
-    // 427 / 228).  A device position is unknown here and counts as 0.
+    // 427 / 228).  A device position is unknown here and counts as 0, and the launch
+    // covers the whole cache: its workgroups past the position, which come and go,
+    // let those with keys meet on the same CUs.  With heads of 128, whose products
+    // that doubles, the matrix form then starts at 256 tokens and 1000000 scores (32 /
+    // 8 heads, caches of 600 and 2600 rows: 128 at 60 25 / 35 us, 160 at 30 25 / 36,
+    // 128 at 100 34 / 42, 200 at 0 32 / 39 and 44 / 46; 256 at 0 42 / 42 and 59 / 57,
+    // at 1000 150 / 102).
     const int64_t pos = a.d_pos ? 0 : std::max(0, std::min(a.pos, a.max_seq));
     const int64_t rows = (int64_t)a.m * rep;
-    if ((a.hd == 128 || a.hd == 64) && a.m > 1 && a.nh * (int64_t)a.m * (2 * pos + a.m) >= 480000 &&
+    const bool far = a.d_pos && a.hd == 128;
+    if ((a.hd == 128 || a.hd == 64) && a.m >= (far ? 256 : 2) &&
+        a.nh * (int64_t)a.m * (2 * pos + a.m) >= (far ? 2000000 : 480000) &&
         ((uintptr_t)a.q & 15u) == 0 && rows <= 65535ll * kMmRows) {
         const int64_t ch = a.d_pos ? a.cmax : std::min<int64_t>(a.cmax, (pos + a.m + kAttnChunk - 1) / kAttnChunk);
         // 64 rows a workgroup (one wave with rows per SIMD) while two workgroups

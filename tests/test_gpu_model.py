@@ -150,7 +150,8 @@ def test_attention_bitexact(nh, nkv, hd, m, pos):
 # KV head, both head sizes, 64 rows a workgroup and (200 queries of 32 heads)
 # 128 rows and several chunks, ragged row blocks and chunks; bad: later tokens
 # hold infinite and NaN values and keys, which earlier queries of the same
-# workgroup do not see
+# workgroup do not see.  The same queries with a device position take the other
+# forms (its matrix form: below)
 @pytest.mark.parametrize("nh,nkv,hd,m,pos", [(32, 8, 128, 70, 300), (4, 2, 64, 300, 200), (3, 1, 128, 250, 500),
                                              (16, 1, 64, 33, 900), (8, 8, 128, 130, 777), (32, 8, 128, 200, 900)])
 @pytest.mark.parametrize("bad", [False, True])
@@ -178,6 +179,41 @@ def test_attention_matrix_form(nh, nkv, hd, m, pos, bad):
             nan = np.isnan(e)
             assert np.isfinite(e).all() != (bad and i >= m // 2) and np.array_equal(np.isnan(o[i]), nan), i
             assert_same(np.where(nan, 0, o[i]).astype(np.float32), np.where(nan, 0, e).astype(np.float32), "query %d" % i)
+
+
+# the same with a device position, which takes the matrix form from more tokens on: 64 and
+# 128 rows a workgroup, 1, 2, 3, 4 and 16 query heads per KV head, and just below the rule.
+# over: the last tokens lie past the cache, under: the first before it (no result), the
+# others are exact
+@pytest.mark.parametrize("nh,nkv,hd,m,pos,mm", [(32, 8, 128, 256, 300, True), (32, 8, 128, 255, 60, False),
+                                                (12, 4, 128, 410, 100, True), (4, 2, 64, 350, 200, True),
+                                                (6, 2, 64, 300, 0, True), (16, 1, 64, 180, 300, True),
+                                                (8, 8, 64, 250, 100, True), (8, 8, 64, 240, 100, False)])
+@pytest.mark.parametrize("where", ["inside", "over", "under"])
+def test_attention_matrix_form_device_position(nh, nkv, hd, m, pos, mm, where):
+    print("attention matrix form, device position", nh, nkv, hd, m, pos, where, flush=True)
+    S = pos + m + 30
+    cache = Cache(nkv, S, hd)
+    _fill_cache(cache, S, seed=nh + m)
+    p = {"inside": pos, "over": S - m + 37, "under": -41}[where]
+    q = np.random.default_rng(pos + m).standard_normal((m, nh * hd)).astype(np.float32)
+    qt = torch.from_numpy(q).to(DEV)
+    d_pos = torch.tensor([p], dtype=torch.int32, device=DEV)
+    out = torch.full((m, nh * hd), 3.0, device=DEV)
+
+    def call():
+        bl.check(bl.lib.btl_attention(qt.data_ptr(), m, nh, ctypes.byref(cache.c), 0, d_pos.data_ptr(), out.data_ptr(),
+                                      None, 0, stream()))
+
+    call()
+    o = out.cpu().numpy()
+    none = [i for i in range(m) if not 0 <= p + i < S]
+    assert len(none) == {"inside": 0, "over": 37, "under": 41}[where]
+    assert np.isnan(o[none]).all() and np.isfinite(np.delete(o, none, 0)).all()
+    host = cache.host()
+    for i in sorted({0, 1, 40, 41, 42, m // 2, m - 39, m - 38, m - 37, m - 2, m - 1} - set(none)):
+        assert_same(o[i], orc.attn_decode(q[i], *host, nh, p + i + 1), "query %d" % i)
+    assert any("k_attn_mm" in f for f in launched(call)) == mm
 
 
 def test_attention_device_position():

@@ -774,14 +774,18 @@ __device__ __forceinline__ float ld_part(const float* p)
 // The chunk merge of one (query, head) by one wave, k_attn_combine's
 // arithmetic: y[d] = (sum_c w_c o_c[d]) / (sum_c w_c l_c), w_c = exp(m_c -
 // max_c m_c), both sums sequential over the chunks.  part: the head's chunk
-// slots of st = hd + 2 floats.  Before the chunk count is known (cfun(): C,
-// or <= 0 for no result -> NaN), the (m, l) of the first 128 slots below cpre
-// and the values of the first 32 are loaded, all in flight together; the values
-// of later chunks follow in two alternating blocks of 16, each loaded while the
-// other is added (read one chunk at a time, every chunk past the first 16 cost
-// a round trip to memory: one token over 6001 keys 41 us, now 24).  SC1: the
-// slots were written by other workgroups of this launch (coherent loads).
-template <bool SC1, typename CF>
+// slots of st = hd + 2 floats.  cfun(): the chunk count C, or <= 0 for no result
+// -> NaN; cpre: C, or the cache's chunks where C is read on the device.  The (m,
+// l) of the first 64 slots below cpre and the values of the first 16 are loaded
+// before C is known, all in flight together; the values of later chunks follow in
+// two alternating blocks of 16, each loaded while the other is added (read one
+// chunk at a time, every chunk past the first 16 cost a round trip to memory: one
+// token over 6001 keys 41 us, now 24).  KNOWN: cpre is C, so the second block and
+// the (m, l) of slots 64 .. 127 start with the first (where C is not known that
+// loads a long cache's unused slots: 32 tokens of 8 heads of 128 in a cache of 2600
+// rows 11.4 -> 12.1 us).  SC1: the slots were written by other workgroups of this
+// launch (coherent loads).
+template <bool SC1, bool KNOWN, typename CF>
 __device__ __forceinline__ void attn_merge_head(const float* part, int st, int cpre, int hd, int lane, float* y,
                                                 CF cfun)
 {
@@ -792,9 +796,15 @@ __device__ __forceinline__ void attn_merge_head(const float* part, int st, int c
     // values are never used): a per-lane or per-slot condition here made the
     // compiler wait for the earlier loads before issuing the (m, l) loads
     const int clast = max(cpre, 1) - 1;
-    const int cl = min(lane, clast), cl2 = min(lane + 64, clast);
-    const float m_pre = ld_part<SC1>(&part[cl * st]), m_pre2 = ld_part<SC1>(&part[cl2 * st]);
-    const float l_pre = ld_part<SC1>(&part[cl * st + 1]), l_pre2 = ld_part<SC1>(&part[cl2 * st + 1]);
+    const int cl = min(lane, clast);
+    const float m_pre = ld_part<SC1>(&part[cl * st]);
+    const float l_pre = ld_part<SC1>(&part[cl * st + 1]);
+    float m_pre2 = 0.0f, l_pre2 = 0.0f;
+    if (KNOWN && clast >= 64) {  // uniform
+        const int cl2 = min(lane + 64, clast);
+        m_pre2 = ld_part<SC1>(&part[cl2 * st]);
+        l_pre2 = ld_part<SC1>(&part[cl2 * st + 1]);
+    }
     float p0[2][kB], p1[2][kB];
     const auto load = [&](int c, int i) {
 #pragma unroll
@@ -806,29 +816,31 @@ __device__ __forceinline__ void attn_merge_head(const float* part, int st, int c
         __builtin_amdgcn_sched_barrier(0);  // all of them issue before the next use
     };
     load(0, 0);
-    if (clast >= kB) load(kB, 1);  // uniform
+    if (KNOWN && clast >= kB) load(kB, 1);  // uniform
     const int C = cfun();
     if (C <= 0) {
         if (h0) y[d0] = __builtin_nanf("");
         if (h1) y[d1] = __builtin_nanf("");
         return;
     }
+    if (!KNOWN && C > kB) load(kB, 1);  // uniform
+    constexpr int kMl = KNOWN ? 128 : 64;  // slots whose (m, l) are loaded
     float M = -__builtin_inff();
     for (int c0 = 0; c0 < C; c0 += 64) {
         const int cc = c0 + lane;
-        const float mv = c0 == 0 ? m_pre : (c0 == 64 ? m_pre2 : (cc < C ? ld_part<SC1>(&part[cc * st]) : 0.0f));
+        const float mv = c0 == 0 ? m_pre : (c0 < kMl ? m_pre2 : (cc < C ? ld_part<SC1>(&part[cc * st]) : 0.0f));
         M = fmaxf(M, wave_max_f32(cc < C ? mv : -__builtin_inff()));
     }
     float L = 0.0f, O0 = 0.0f, O1 = 0.0f;
     for (int c0 = 0; c0 < C; c0 += 64) {
         const int cc = c0 + lane;
         float mv = m_pre, lv = l_pre;
-        if (c0 == 64) {
-            mv = m_pre2;
-            lv = l_pre2;
-        } else if (c0 > 64) {
+        if (c0 >= kMl) {
             mv = cc < C ? ld_part<SC1>(&part[cc * st]) : 0.0f;
             lv = cc < C ? ld_part<SC1>(&part[cc * st + 1]) : 0.0f;
+        } else if (c0 > 0) {
+            mv = m_pre2;
+            lv = l_pre2;
         }
         const float w = cc < C ? btl_expf_below(__fsub_rn(mv, M)) : 0.0f;
         const float l = cc < C ? lv : 0.0f;
@@ -1006,15 +1018,15 @@ __global__ __launch_bounds__(1024) void k_attn_dec1(AttnArgs a, DecKv kv)
         __syncthreads();
         if (!s_last) return;
         const int C = (T + kAttnChunk - 1) / kAttnChunk;
-        attn_merge_head<true>(a.part + (int64_t)h * a.cmax * (hd + 2), hd + 2, C, hd, lane, a.out + (int64_t)h * hd,
+        attn_merge_head<true, true>(a.part + (int64_t)h * a.cmax * (hd + 2), hd + 2, C, hd, lane, a.out + (int64_t)h * hd,
                               [C]() { return C; });
     }
 }
 
 // grid (m, nh), block 64: y[d] = (sum_c w_c o_c[d]) / (sum_c w_c l_c),
-// w_c = exp(m_c - max_c m_c), both sums sequential over the chunks.  Lane c
-// holds chunk c's (m_c, l_c); the value loads of up to 16 chunks are all in
-// flight before the sums.
+// w_c = exp(m_c - max_c m_c), both sums sequential over the chunks
+// (attn_merge_head).  DEV: the position is read on the device.
+template <bool DEV>
 __global__ __launch_bounds__(64) void k_attn_combine(AttnArgs a)
 {
     const int i = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
@@ -1029,8 +1041,8 @@ __global__ __launch_bounds__(64) void k_attn_combine(AttnArgs a)
     // slots past the query's chunks are not loaded where the host knows the
     // position (the 512-token prompt in a cache of 16 chunks, 4.5 of them in use
     // on average: 24.5 -> 14.3 us)
-    const int cpre = a.d_pos ? a.cmax : count(a.pos);
-    attn_merge_head<false>(part, st, cpre, hd, lane, y, [&]() { return a.d_pos ? count(*a.d_pos) : cpre; });
+    const int cpre = DEV ? a.cmax : count(a.pos);
+    attn_merge_head<false, !DEV>(part, st, cpre, hd, lane, y, [&]() { return DEV ? count(*a.d_pos) : cpre; });
 }
 
 // k_attn_combine for one token: grid (nh, ceil(hd / 16)), block 256.  A workgroup
@@ -1223,7 +1235,9 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t st)
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (a.m == 1) return launch_combine1(a, st);
-    hipLaunchKernelGGL(k_attn_combine, dim3((unsigned)a.m, (unsigned)a.nh), dim3(64), 0, st, a);
+    const dim3 gc((unsigned)a.m, (unsigned)a.nh);
+    if (a.d_pos) hipLaunchKernelGGL(k_attn_combine<true>, gc, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL(k_attn_combine<false>, gc, dim3(64), 0, st, a);
     return hipGetLastError();
 }
 

@@ -181,6 +181,40 @@ def test_attention_matrix_form(nh, nkv, hd, m, pos, bad):
             assert_same(np.where(nan, 0, o[i]).astype(np.float32), np.where(nan, 0, e).astype(np.float32), "query %d" % i)
 
 
+# the merge of many chunks: around its blocks of 16 chunks and 64 (m, l) pairs, the last
+# query in chunk number `chunks`, host and device position, and one token whose chunks are
+# merged in its launch (a device position estimated as 0)
+@pytest.mark.parametrize("chunks", [15, 16, 17, 32, 33, 48, 64, 65, 96, 97, 128, 129, 140])
+@pytest.mark.parametrize("nh,nkv,hd,m", [(2, 1, 128, 3), (3, 3, 64, 40), (2, 1, 48, 2)])
+def test_attention_merge_of_many_chunks(nh, nkv, hd, m, chunks):
+    print("attention merge", nh, nkv, hd, m, chunks, flush=True)
+    T, S = 64 * chunks - 61 + m // 2, 64 * chunks + 200  # queries on both sides of a chunk's first key
+    pos = T - m
+    cache = Cache(nkv, S, hd)
+    _fill_cache(cache, S, seed=nh + chunks)
+    rng = np.random.default_rng(chunks)
+    q, k, v = (rng.standard_normal((m, n * hd)).astype(np.float32) for n in (nh, nkv, nkv))
+    qt, kt, vt = (torch.from_numpy(a).to(DEV) for a in (q, k, v))
+    host = cache.host()
+    exp = {i: orc.attn_decode(q[i], *host, nh, pos + i + 1) for i in {0, m // 2, m - 1}}
+    out = torch.empty((m, nh * hd), device=DEV)
+    for d_pos in (None, torch.tensor([pos], dtype=torch.int32, device=DEV)):
+        out.fill_(3.0)
+        bl.check(bl.lib.btl_attention(qt.data_ptr(), m, nh, ctypes.byref(cache.c), 0 if d_pos is not None else pos,
+                                      d_pos.data_ptr() if d_pos is not None else None, out.data_ptr(), None, 0,
+                                      stream()))
+        for i, e in exp.items():
+            assert_same(out[i], e, "query %d" % i)
+    cos, sin, dc, ds = rope_dev(500000.0, hd, S)
+    for _ in range(2):  # the counters are back at zero
+        out.fill_(3.0)
+        bl.check(bl.lib.btl_rope_append_attention(qt.data_ptr(), kt.data_ptr(), vt.data_ptr(), 1, nh,
+                                                  ctypes.byref(cache.c), 0, d_pos.data_ptr(), dc.data_ptr(),
+                                                  ds.data_ptr(), out.data_ptr(), None, 0, stream()))
+        qr = orc.rope_apply(q[0].reshape(nh, hd), cos[pos], sin[pos]).reshape(-1)
+        assert_same(out[0], orc.attn_decode(qr, *cache.host(), nh, pos + 1), "one token")
+
+
 # the same with a device position, which takes the matrix form from more tokens on: 64 and
 # 128 rows a workgroup, 1, 2, 3, 4 and 16 query heads per KV head, and just below the rule.
 # over: the last tokens lie past the cache, under: the first before it (no result), the
@@ -270,9 +304,10 @@ def test_rope_append_attention_one_token(nh, nkv, hd, pos, dpos, merge, tune):
 
 @pytest.mark.parametrize("pos", [4095, 8190])
 def test_rope_append_attention_one_token_long_cache(pos, tune):
-    # more than 64 key chunks (the merge walks them in several 64-chunk passes),
-    # Llama-3-8B head layout; then repeated calls (the merge counters must be
-    # back at zero after each launch) and a device position outside the cache
+    # more than 64 key chunks, Llama-3-8B head layout, merged in the launch (the
+    # position is estimated as 0) and in a second one; repeated calls (the merge
+    # counters must be back at zero after each launch) and a device position
+    # outside the cache
     nh, nkv, hd, S = 32, 8, 128, 8192
     print("rope_append_attention long", pos, flush=True)
     rng = np.random.default_rng(pos)
@@ -313,7 +348,7 @@ def test_rope_append_attention_one_token_merge_sequence(nh, nkv, hd, tune):
     # The merge in the launch over a sequence of calls on one caller workspace:
     # falling and rising positions (the workspace keeps the partials of earlier
     # calls), the workspace overwritten with other bits between some calls,
-    # more key chunks than the merge loads ahead (16), the last call repeated;
+    # more key chunks than the merge loads ahead (32), the last call repeated;
     # the counters must be back at zero after every launch, each call against
     # the oracle.
     print("rope_append_attention sequence", nh, nkv, hd, flush=True)

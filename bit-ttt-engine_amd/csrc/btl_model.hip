@@ -1726,14 +1726,41 @@ __global__ __launch_bounds__(256) void k_dense_gemv(const void* w, int64_t n, in
     }
 }
 
+// Few outputs: a wave each (k_dense_gemv, m rows) instead of k_dense_mm, whose one
+// workgroup per tile walks all of k however small the output is.  Measured, us, a
+// wave per output / matrix form:
+//   f32, below 12 MB of weights: k = 4096, n = 256, 4096 outputs 6.2 / 7.4, 5120 7.1 /
+//     7.3, 6912 9.0 / 7.4; k = n = 512, 5120 3.2 / 3.5, 6144 3.8 / 3.5; more (read once
+//     per token row): k = 4096, n = 1024, 2048 6.6 / 7.3, 3072 8.0 / 7.4; long k: 8192,
+//     n = 128, 4096 9.8 / 11.7, n = 512, 3072 11.2 / 11.8, 4096 14.4 / 11.9, 14336, n =
+//     128, 3968 18.0 / 18.6
+//   bf16: k = 4096 (its row in registers), n = 1024, 6144 7.7 / 8.2, n = 2048, 4096 8.2 /
+//     8.6, 6144 10.5 / 8.6; k = 512, n = 512, 5120 3.4 / 3.5, 6144 4.1 / 3.5; k = 8192, n =
+//     512, 2560 13.2 / 13.7, 4096 14.4 / 13.7; k = 14336, n = 128, 2048 27 / 22
+//   a k that ends within a step of 2048 elements costs a whole one: 3000, n = 900,
+//     f32 1800 5.3 / 6.4, 2700 7.0 / 6.4, bf16 1800 8.4 / 7.0
+static bool dense_few(int wkind, int64_t n, int64_t k, int64_t m)
+{
+    const int64_t outs = m * n;
+    if (outs > 6144) return false;
+    const int64_t mb = n * k * (wkind == XK_BF16 ? 2 : 4) >> 20;
+    const bool whole = k <= 2048 || k % 2048 == 0;
+    if (wkind == XK_BF16) {
+        if (!whole || k > 8192) return false;
+        return outs <= (k == 4096 ? (mb <= 8 ? 6144 : 4096) : (k <= 2048 ? 5120 : 2560));
+    }
+    if (!whole) return outs <= 2048;
+    return outs <= (k > 4096 ? (mb < 12 ? 4096 : 3072) : (mb < 12 ? 5120 : 2048));
+}
+
 hipError_t launch_dense_gemv(const void* w, int wkind, int64_t n, int64_t k, const float* x, int64_t m, float* y,
                              hipStream_t st)
 {
     if (n < 1 || m < 1 || m > 65535 || k < 4 || k % 4 || k > INT32_MAX / 2) return hipErrorInvalidValue;
-    // one token row: each weight is used once, streamed through registers; from
-    // two on the matrix form reads the weights once per 16 or 32 rows (n = 5632,
-    // k = 4096, f32, us: m = 1 17 / 22, 2 29 / 22)
-    if (m >= 2 && k <= kDenseMmMaxK && (n + 15) / 16 * ((m + 15) / 16) <= kDenseMmMaxTiles)
+    // one token row: each weight is used once, streamed through registers; from two
+    // on the matrix form reads the weights once per 16 or 32 rows (n = 5632, k =
+    // 4096, f32, us: m = 1 17 / 22, 2 29 / 22)
+    if (m >= 2 && !dense_few(wkind, n, k, m) && k <= kDenseMmMaxK && (n + 15) / 16 * ((m + 15) / 16) <= kDenseMmMaxTiles)
         return launch_dense_mm(w, wkind, n, k, x, m, y, st);
     const unsigned G = (unsigned)std::min<int64_t>((n + 3) / 4, 1024);
     const dim3 grid(G, (unsigned)m), block(256);

@@ -1060,12 +1060,14 @@ def test_dense_linear(n, k, m, dt):
     assert np.abs(y.cpu().numpy() - ref).max() <= 1e-4 * max(1.0, np.abs(ref).max())
 
 
-# several token rows: the matrix form, in tiles of 16 x 16 and (from 160 of
-# them) 32 x 32 outputs; rows shorter than a block of 256 elements, a row of
+# several token rows: a wave per output for few of them, else the matrix form, in
+# tiles of 16 x 16 and (from 160 of them) 32 x 32 outputs; rows shorter than a block of 256 elements, a row of
 # blocks only, and last chunks that end inside a wave's and between the waves'
 # chains; ragged token and row tiles
 @pytest.mark.parametrize("n,k,m", [(33, 4, 2), (17, 252, 3), (70, 260, 17), (40, 1028, 64), (129, 768, 33),
-                                   (50, 4100, 16), (2570, 516, 40), (1030, 256, 130), (2590, 1532, 65)])
+                                   (50, 4100, 16), (2570, 516, 40), (1030, 256, 130), (2590, 1532, 65),
+                                   (2570, 4, 2), (1717, 252, 3), (310, 260, 17), (90, 1028, 64), (161, 768, 33),
+                                   (330, 4100, 16)])
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 def test_dense_linear_matrix_form(n, k, m, dt):
     print("dense_linear matrix form", n, k, m, dt, flush=True)
@@ -1088,6 +1090,32 @@ def test_dense_linear_matrix_form(n, k, m, dt):
     got = y.cpu().numpy()
     assert np.array_equal(np.isnan(got), nan) and not nan[0].any() and not np.isfinite(exp[1]).any()
     assert np.array_equal(np.where(nan, 0, got).view(np.uint32), np.where(nan, 0, exp).view(np.uint32))
+
+
+# few outputs go a wave each, by their number, the weights' size and the length of a row
+@pytest.mark.parametrize("dt,n,k,m,mm", [("f32", 256, 4096, 20, False), ("f32", 257, 4096, 20, True),
+                                         ("f32", 1024, 4096, 2, False), ("f32", 1024, 4096, 3, True),
+                                         ("f32", 1024, 3000, 2, False), ("f32", 1024, 3000, 3, True),
+                                         ("f32", 64, 14336, 64, False), ("f32", 64, 14336, 65, True),
+                                         ("f32", 512, 8192, 6, False), ("f32", 512, 8192, 7, True),
+                                         ("bf16", 256, 4096, 24, False), ("bf16", 256, 4096, 25, True),
+                                         ("bf16", 2048, 4096, 2, False), ("bf16", 2048, 4096, 3, True),
+                                         ("bf16", 128, 8192, 20, False), ("bf16", 128, 8192, 21, True),
+                                         ("bf16", 512, 2048, 10, False), ("bf16", 512, 2048, 11, True),
+                                         ("bf16", 16, 3000, 2, True), ("bf16", 16, 14336, 2, True),
+                                         ("f32", 16, 64, 1, False), ("f32", 16, 64, 2, False)])
+def test_dense_linear_launches(dt, n, k, m, mm):
+    print("dense_linear launches", dt, n, k, m, flush=True)
+    x = torch.randn((m, k), device=DEV)
+    w = torch.randn((n, k), device=DEV).to(torch.bfloat16 if dt == "bf16" else torch.float32)
+    y = torch.empty((m, n), device=DEV)
+    code = bl.BTL_BF16 if dt == "bf16" else bl.BTL_F32
+    names = launched(lambda: bl.check(bl.lib.btl_dense_linear(w.data_ptr(), code, n, k, x.data_ptr(), m, y.data_ptr(),
+                                                              stream())))
+    assert len(names) == 1 and ("k_dense_mm" in names[0]) == mm
+    exp = orc.dense_linear(x.cpu().numpy()[-2:], w.view(torch.int16).cpu().numpy().view(np.uint16) if dt == "bf16"
+                           else w.cpu().numpy())
+    assert_same(y[-2:], exp)
 
 
 def test_decoder_dense_head_matches_oracle():

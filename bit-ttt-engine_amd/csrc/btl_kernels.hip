@@ -3215,6 +3215,22 @@ static void launch_ref_st(dim3 grid, hipStream_t st, const void* x, int64_t m, i
     hipLaunchKernelGGL((k_ref_f32_st<XK, YK, kRefDepth, KX, TR>), grid, dim3(256), 0, st, x, m, k, g, tx);
 }
 
+// From 8 token rows and 65536 outputs on the f32 matrix instructions are faster (us,
+// the staged form / that one: q|k|v at m = 8 17 / 20, 16 30 / 26, 32 55 / 33; down at
+// m = 8 51 / 59, 16 100 / 77; gate|up at m = 8 61 / 52, 16 118 / 76): below them a
+// 16-token tile is mostly padding.  Just above them the staged form's workgroups (two
+// tokens x 32 rows) still fit the chip once, and for k of 2048 to 4096 its time then
+// is the shorter one: n = 4096, m = 16 (1024 workgroups), k = 1536 10.9 / 10.8, 2048
+// 12.5 / 13.3, 4096 19.6 / 23.7, 5632 39 / 31 (a token's row no longer fits 16 KB of
+// LDS); at k = 4096 also where a second token tile is mostly padding: n = 4096, m = 17
+// and 20 (1280) 22.1 / 23.9 and 23.3 / 23.9, 22 (1408) 26.8 / 23.8; n = 6144, two tiles
+// of waves, m = 17 (1728) 29.4 / 31.8, 20 (1920) 34.5 / 31.2.
+static bool ref_staged_small(int64_t m, int64_t k, int64_t wgs, int64_t tiles)
+{
+    if (k < 2048 || k > 4096) return false;
+    return wgs <= 1024 || (k > 3072 && m > 16 && wgs <= (tiles > 512 ? 1728 : 1280));
+}
+
 hipError_t launch_ref_f32_group(const void* x, int xkind, int64_t m, int64_t k, const uint8_t* const* w,
                                 const int64_t* n, const float* scale, void* const* y, int count, int ykind,
                                 hipStream_t st, int xf, const RefXf* t)
@@ -3242,6 +3258,7 @@ hipError_t launch_ref_f32_group(const void* x, int xkind, int64_t m, int64_t k, 
     RefGroup g{};
     g.count = count;
     int b = 0;
+    int64_t row_tiles = 0;
     for (int i = 0; i < count; ++i) {
         g.w[i] = w[i];
         g.y[i] = y[i];
@@ -3249,13 +3266,10 @@ hipError_t launch_ref_f32_group(const void* x, int xkind, int64_t m, int64_t k, 
         g.n[i] = n[i];
         g.wg_begin[i] = b;
         b += (int)((n[i] + rows - 1) / rows);
+        row_tiles += (n[i] + 15) / 16;
     }
     g.wg_begin[count] = b;
-    // from 8 token rows and 65536 outputs on the f32 matrix instructions are
-    // faster (us, this form / that one: q|k|v at m = 8 17 / 20, 16 30 / 26, 32 55
-    // / 33; down at m = 8 51 / 59, 16 100 / 77; gate|up at m = 8 61 / 52, 16 118 /
-    // 76): below them a 16-token tile is mostly padding
-    if (xf == 0 && m >= 8 && m * n_total >= 65536)
+    if (xf == 0 && m >= 8 && m * n_total >= 65536 && !ref_staged_small(m, k, b * ((m + 1) / 2), row_tiles * ((m + 15) / 16)))
         return launch_ref_mm(x, xkind, m, k, g, ykind, st);
     // two token rows per workgroup from m = 2 on (the weight chunk's read and
     // coefficient lookup shared; x of both rows in LDS: at most 2 x 64 KB)

@@ -11,6 +11,7 @@ import torch
 
 import bitlinear as bl
 from datagen import activations, random_codes, ternary, weights
+from launches import launched
 from oracle import oracle as orc
 
 pytestmark = [pytest.mark.gpu,
@@ -711,7 +712,8 @@ def test_linear_f32_ref_staged_form(m, k, n, xdt, ydt):
 # and with eight), with ragged token and row tiles, a group of layers, fewer
 # 32-input blocks than are in flight (k = 64) and a remainder of them (k = 320)
 REF_MM_CASES = [(17, 192, (4000,)), (17, 64, (4000, 33)), (33, 320, (5000,)), (65, 64, (4968, 33)),
-                (65, 4096, (1100,)), (128, 320, (8000,)), (100, 64, (8190, 17, 33)), (8, 128, (8192,))]
+                (65, 4096, (1100,)), (65, 4096, (1500,)), (128, 320, (8000,)), (100, 64, (8190, 17, 33)),
+                (8, 128, (8192,))]
 
 
 @pytest.mark.parametrize("m,k,ns", REF_MM_CASES)
@@ -737,6 +739,25 @@ def test_linear_f32_ref_matrix_form(m, k, ns, xdt, ydt):
             assert_f32_identical(y, yr)
         else:
             assert_bf16_matches(y, yr)
+
+
+# which form many token rows take: just above the matrix form's least outputs the staged
+# form still fits the chip once
+@pytest.mark.parametrize("m,k,n,mm", [(16, 4096, 4095, False), (16, 1984, 4096, True), (16, 2048, 4096, False),
+                                      (17, 2048, 4096, True), (16, 3072, 4096, False), (17, 3072, 4096, True),
+                                      (16, 4096, 4096, False), (16, 4160, 4096, True), (20, 4096, 4096, False),
+                                      (21, 4096, 4096, True), (11, 4096, 6144, True), (17, 4096, 6144, False),
+                                      (19, 4096, 6144, True), (7, 64, 12800, False), (8, 64, 12800, True)])
+def test_linear_f32_ref_launches(m, k, n, mm):
+    print("f32 ref launches", m, k, n, flush=True)
+    x = activations(m, k, seed=m + k)
+    wb = random_codes(n, k, seed=n, p3=0.1)
+    pt = bl.PackedTensor(torch.from_numpy(wb).to(DEV), 0.0173, (n, k), DEV)
+    xt, ys = to_dev(x, torch.float32), []
+    names = launched(lambda: ys.append(bl.BitLinearHip.forward(xt, pt, mode="f32_ref")))
+    assert len(names) == 1 and ("k_ref_mm" in names[0]) == mm
+    rows = [0, m - 1]
+    assert_f32_identical(ys[0][rows], orc.forward_f32(x[rows], wb, n, np.float32(0.0173)))
 
 
 # special inputs in the reference's order: subnormal inputs and partial sums

@@ -3437,8 +3437,8 @@ hipError_t launch_ref_seq(const void* x, int xkind, int64_t m, int64_t k, const 
 }
 
 // ---------------------------------------------------------------------------
-// k_generic_i8: one wave per output, any k % 4 == 0, any alignment (the sizes
-// that k_rag_i8's 32-bit offsets do not reach)
+// k_generic_i8: one wave per output, any k % 4 == 0, any alignment: few outputs
+// of a short k, and rows longer than k_rag_i8's 32-bit offsets reach
 // ---------------------------------------------------------------------------
 template <int YK>
 __global__ __launch_bounds__(256) void k_generic_i8(const int8_t* q, const float* xs, int64_t m,
@@ -3616,13 +3616,17 @@ hipError_t launch_generic_i8(const int8_t* q, const float* xs, int64_t m, int64_
 {
     const int64_t outs = m * n;
     if (outs <= 0) return hipSuccess;
-    // the matrix form wherever its 32-bit offsets reach (64 rows of k bytes; at
-    // most 2^24 workgroups of 256 threads)
-    if (k >= 4 && k < (1 << 24) && ((m + 15) / 16) * ((n + 15) / 16) < (1 << 24)) {
-        const RagArgs a{q, xs, w, sw, y, acc_out, n, (int)m, (int)k};
+    // the matrix form wherever its 32-bit offsets reach (32 rows of k bytes), but for
+    // few outputs of a short k, where its sums' way through LDS costs more than the
+    // products (with the quantiser, us, a wave per output / this: k = 100, n = 257, m =
+    // 1 4.51 / 4.64, 8 4.96 / 5.08, 16 5.20 / 5.17; k = 1004, n = 257, m = 1 6.3 / 4.8)
+    if (k >= 4 && k < (1 << 24) && !(k < 256 && outs <= 3072)) {
         // 32 x 32 tiles when they fill the chip, else 16 x 16 (256 tokens, k = 4092,
         // n = 4096: 24 / 43 us; 77, 3252, 1001: both under a launch and its call)
         const bool big = ((m + 31) / 32) * ((n + 31) / 32) >= 256;
+        const int t = big ? 32 : 16;
+        if (((m + t - 1) / t) * ((n + t - 1) / t) >= (1 << 24)) return hipErrorInvalidValue;  // of 256 threads: below 2^32
+        const RagArgs a{q, xs, w, sw, y, acc_out, n, (int)m, (int)k};
 #define BTL_RAG(YKV)                                  \
     if (big) launch_rag_t<YKV, 2, 2>(a, st);          \
     else launch_rag_t<YKV, 1, 1>(a, st);
@@ -3634,6 +3638,7 @@ hipError_t launch_generic_i8(const int8_t* q, const float* xs, int64_t m, int64_
         return hipGetLastError();
 #undef BTL_RAG
     }
+    if ((outs + 3) / 4 >= (1 << 24)) return hipErrorInvalidValue;
     dim3 grid((unsigned)((outs + 3) / 4));
     if (ykind == YK_BF16)
         hipLaunchKernelGGL(k_generic_i8<YK_BF16>, grid, dim3(256), 0, st, q, xs, m, k, w, n, sw, y, acc_out);

@@ -626,9 +626,10 @@ def test_large_m_sampled_rows():
 # rows that are no multiple of 16 bytes long, weights and int8 tokens starting
 # at any byte: rows shorter than a dword and than a segment of 256 weights, a
 # last group that is full, partial and empty, tiles of 16 x 16 and (256 of
-# them) 32 x 32 outputs with ragged edges
+# them) 32 x 32 outputs with ragged edges; up to 3072 outputs of less than 256
+# weights go a wave each
 @pytest.mark.parametrize("m,k,n", [(1, 4, 1), (5, 4, 33), (17, 100, 70), (64, 252, 31), (2, 260, 16), (33, 3252, 129),
-                                   (515, 516, 490)])
+                                   (515, 516, 490), (94, 4, 33), (44, 100, 70), (97, 252, 32), (513, 4, 520)])
 @pytest.mark.parametrize("off", [0, 1, 2, 3])
 def test_linear_i8_ragged_matrix_form(m, k, n, off):
     print("i8 ragged", m, k, n, off, flush=True)
@@ -648,6 +649,27 @@ def test_linear_i8_ragged_matrix_form(m, k, n, off):
     y = bl.linear_i8(qb[off:].view(m, k), torch.from_numpy(s).to(DEV), pt, acc_out=acc)
     assert np.array_equal(acc.cpu().numpy(), accr)
     assert_f32_identical(y, yr)
+
+
+# a wave per output for few outputs of a short k, and for rows past the 32-bit offsets of
+# the matrix form
+@pytest.mark.parametrize("m,k,n,waves", [(1, 4, 1, True), (12, 252, 256, True), (12, 252, 257, False), (8, 260, 256, False),
+                                         (2, (1 << 24) - 4, 3, False), (2, 1 << 24, 3, True)])
+def test_linear_i8_ragged_launches(m, k, n, waves):
+    print("i8 ragged launches", m, k, n, flush=True)
+    x = activations(m, k, seed=m)
+    wb = random_codes(n, k, seed=n, p3=0.1)
+    buf = torch.zeros(wb.size + 1, dtype=torch.uint8, device=DEV)
+    buf[1:] = torch.from_numpy(wb).to(DEV)
+    pt = bl.PackedTensor(buf[1:], 0.0123, (n, k), DEV)
+    yr, q, s, accr = orc.forward_i8(x, wb, n, np.float32(0.0123))
+    acc = torch.full((m, n), 7, dtype=torch.int32, device=DEV)
+    qt, st = torch.from_numpy(np.ascontiguousarray(q)).to(DEV).view(m, k), torch.from_numpy(s).to(DEV)
+    ys = []
+    names = launched(lambda: ys.append(bl.linear_i8(qt, st, pt, acc_out=acc)))
+    assert len(names) == 1 and ("k_generic_i8" in names[0]) == waves
+    assert np.array_equal(acc.cpu().numpy(), accr)
+    assert_f32_identical(ys[0], yr)
 
 
 # --- reference fp32 semantics ---------------------------------------------------------

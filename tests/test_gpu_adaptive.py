@@ -101,11 +101,14 @@ def test_adaptive_linear_output_over_its_input(m, nb, n, k):
     arr = (ctypes.POINTER(bl.BtlPacked) * nb)(*[ctypes.pointer(c) for c in cs])
     x = activations(m, k, seed=m)
     e = orc.adaptive_forward_i8(x, packed, s, n)
+    need = bl.lib.btl_adaptive_workspace_bytes(m, n, k, nb)
+    ws = torch.empty((need,), dtype=torch.uint8, device=DEV)
     for row in (0, 1):
         buf = torch.zeros((m * max(n, k) + k,), device=DEV)
         buf[:m * k] = torch.from_numpy(x).to(DEV).reshape(-1)
         y = buf[row * k:row * k + m * n]
-        bl.check(bl.lib.btl_adaptive_linear(arr, nb, buf.data_ptr(), bl.BTL_F32, m, k, y.data_ptr(), bl.BTL_F32, None, 0,
+        bl.check(bl.lib.btl_adaptive_linear(arr, nb, buf.data_ptr(), bl.BTL_F32, m, k, y.data_ptr(), bl.BTL_F32,
+                                            ws.data_ptr(), need,
                                             ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
         assert np.array_equal(y.cpu().numpy().reshape(m, n).view(np.uint32), e.view(np.uint32)), row
 
@@ -114,7 +117,7 @@ def test_adaptive_linear_output_over_its_input(m, nb, n, k):
 # launch where its tiles would be padding.  Columns checked: the first and last 200
 @pytest.mark.parametrize("m,k,nb,one", [(1, 64, 3, False), (2, 1024, 2, False), (3, 1024, 2, True), (4, 1088, 3, False),
                                         (16, 1088, 3, False), (17, 1088, 3, True), (17, 1088, 4, False),
-                                        (32, 3136, 2, False), (64, 1088, 4, False), (65, 1088, 4, True)])
+                                        (32, 3136, 2, False), (33, 1088, 4, False), (65, 1088, 4, True)])
 def test_adaptive_linear_few_tokens_of_a_wide_layer(m, k, nb, one):
     print("adaptive few tokens", m, k, nb, flush=True)
     n = 25601

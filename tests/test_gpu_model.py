@@ -234,10 +234,12 @@ def test_attention_matrix_form_device_position(nh, nkv, hd, m, pos, mm, where):
     qt = torch.from_numpy(q).to(DEV)
     d_pos = torch.tensor([p], dtype=torch.int32, device=DEV)
     out = torch.full((m, nh * hd), 3.0, device=DEV)
+    need = bl.lib.btl_attention_workspace_bytes(m, nh, ctypes.byref(cache.c))
+    ws = torch.empty((need,), dtype=torch.uint8, device=DEV)
 
     def call():
         bl.check(bl.lib.btl_attention(qt.data_ptr(), m, nh, ctypes.byref(cache.c), 0, d_pos.data_ptr(), out.data_ptr(),
-                                      None, 0, stream()))
+                                      ws.data_ptr(), need, stream()))
 
     call()
     o = out.cpu().numpy()

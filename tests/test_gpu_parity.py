@@ -72,6 +72,26 @@ def test_quantize_act_bitexact(dtype, m, k):
     assert_f32_identical(s, sr)
 
 
+# every length of the vector form (rows of up to 1024, 4096 and 8192 elements kept in
+# registers, longer ones read twice), each ending in the middle of a round, and rows that are
+# not aligned for it
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [1024, 1028, 3252, 4096, 4100, 6004, 8192, 8196, 20000])
+@pytest.mark.parametrize("off", [0, 1])
+def test_quantize_act_row_lengths(dtype, k, off):
+    print("quantize rows", dtype, k, off, flush=True)
+    m = 3
+    x = activations(m, k, seed=k)
+    x[1, -1], x[2, k - 5] = 31.0, -29.0  # the row's maximum in its last, partial round
+    buf = torch.zeros((m * k + off,), dtype=dtype, device=DEV)
+    buf[off:] = to_dev(x, dtype).reshape(-1)
+    xt = buf[off:].view(m, k)
+    q, s = bl.quantize_act(xt)
+    qr, sr = orc.quantize_act(host_x(xt))
+    assert np.array_equal(q.cpu().numpy(), qr)
+    assert_f32_identical(s, sr)
+
+
 # --- W1.58-A8 linear -------------------------------------------------------------
 
 I8_SHAPES = [

@@ -354,7 +354,8 @@ int add_resid(const Layer& l, const float* resid, int64_t m, hipStream_t st)
 }
 
 // W1.58-A8 contraction of `count` layers sharing one input.
-//   any k % 4 == 0 / any alignment .... quantise into scratch, k_generic_i8
+//   any k % 4 == 0 / any alignment .... quantise into scratch, k_rag_i8 (few
+//                                        outputs: k_generic_i8)
 //   m <= 4 (decode) ................... k_gemv_dec, quantisation fused
 //   otherwise (batched decode, prefill)  quantise in operand order into the
 //                                        workspace, one (split-K) launch of
@@ -383,7 +384,7 @@ int run_i8(const Layer* layers, int count, const void* x, int xkind, const float
     hipError_t e;
 
     if (!fast) {
-        // any k % 4 == 0 / any alignment: quantise once into scratch, one wave per output
+        // any k % 4 == 0 / any alignment: quantise once into scratch, a launch per layer
         const bool scratch = xkind != btl::XK_I8;
         const WsLayout L = ws_layout(m, k, 0);
         void* ws = nullptr;
@@ -449,7 +450,8 @@ int run_i8(const Layer* layers, int count, const void* x, int xkind, const float
     // Batched decode of KN_GEMV_TR_MIN_M .. KN_GEMV_TR_MAX_M token rows (up to
     // 16 rows only from k = KN_GEMV_TR_K16 on): the token-register kernel
     // (bf16 / f32 input, no transform), tokens quantised straight into its
-    // register layout; its K splits (k > 4096) are added in the launch, so it
+    // register layout (calls with a transform, whose quantiser does not write
+    // it, take the routes below); its K splits (k > 4096) are added in the launch, so it
     // needs this workspace's merge counters (else the routes below).  Measured
     // on MI355X, Llama-3-8B MLP, us per call with the quantiser launch:
     // gate|up (k = 4096) at m = 17..32 15.7-16.1 against 19.5-21.0 through

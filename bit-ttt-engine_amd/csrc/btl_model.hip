@@ -492,12 +492,12 @@ __global__ __launch_bounds__(1024) void k_attn_part_g(AttnArgs a)
 // multiply-adds, so the chains over d of the scores and over j of the values
 // are those of attn_chunk_query, bit for bit.  A row is a (query, head of the
 // KV head's group) pair, row rho = query * rep + head; wave w of a workgroup
-// takes the 16 rows at 16 (8 blockIdx.z + w) against the 64-key chunk that the
-// workgroup dequantises into LDS.
+// takes the 16 rows at wg_rows blockIdx.z + 16 w (64 rows a workgroup: the first
+// four waves only) against the 64-key chunk that the workgroup dequantises into LDS.
 //   scores: A = keys (16 at a time), B = rows, so lane 16 q + r ends with the
 //     scores of row r at keys 16 t + 4 q + v (t, v < 4).  Lane 16 q + r holds
-//     q[row r][4 i + q] of every step i in registers for the whole kernel; a
-//     key row sits in LDS as [q][i], four steps per 16-byte read.
+//     q[row r][4 i + q] of every step i in registers, read again for every
+//     chunk; a key row sits in LDS as [q][i], four steps per 16-byte read.
 //   softmax: the maximum and the pairwise sum of a row over its four lanes and
 //     16 registers, in attn_chunk_query's tree.
 //   values: A = rows, B = V.  The probabilities reach the A layout (lane 16 q +
@@ -512,10 +512,10 @@ __global__ __launch_bounds__(1024) void k_attn_part_g(AttnArgs a)
 // chunk's codes are loaded during the values' products and waited for before
 // the partials' stores, which would otherwise stand in front of them in vmcnt.
 //
-// What bounds it: the f32 matrix instructions fill half of its cycles, the
-// softmax and the dequantisation about a quarter; 128 registers at four waves
+// What bounds it: the f32 matrix instructions fill 55 % of its cycles, the other
+// vector instructions (softmax, dequantisation) 23 %; 128 registers at four waves
 // per SIMD leave no room to run a wave's softmax beside its products.  512
-// queries over 2048 keys (32 / 8 heads of 128), us: k_attn_part_g 419 -> 170.
+// queries over 2048 keys (32 / 8 heads of 128), us: k_attn_part_g 419 -> 192.
 constexpr int kMmRows = 128;             // rows per workgroup, 16 a wave
 constexpr int kMmVs = kAttnMaxHd + 16;  // LDS value row stride: the four keys of a step on different banks
 
@@ -1204,7 +1204,8 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t st)
         // 64 rows a workgroup (one wave with rows per SIMD) while two workgroups
         // per CU hold the launch, then 128 rows, then several chunks a workgroup
         // (512 over 2048: 222 us with 512 workgroups, 228 with 1024, 237 with one
-        // chunk each; 256 over 756, 768 workgroups: 58 with one each, 65 with two)
+        // chunk each; 128 to 256 queries of 32 / 8 heads, with one each / with two: 768
+        // workgroups 58 / 65, 800 67.0 / 65.2, 832 66.7 / 65.2, 1024 70 / 68)
         constexpr int64_t kResident = 512;
         const int wg_rows = a.nkv * ((rows + 63) / 64) * ch <= kResident ? 64 : kMmRows;
         const int64_t zb = (rows + wg_rows - 1) / wg_rows;

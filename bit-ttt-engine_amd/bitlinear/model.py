@@ -201,7 +201,7 @@ class BitLlamaHip:
         self._ws_n = need
         self.pos = 0
         self.graph = None
-        self._graph_until = 0  # the position from which decode_steps captures anew
+        self._expect = 0  # where a captured step will mostly run, if past self.pos
 
     # ------------------------------------------------------------------ steps
     def _stream(self):
@@ -348,6 +348,7 @@ class BitLlamaHip:
             cache.reset()
         self.pos = 0
         self.graph = None
+        self._expect = 0
 
     def forward_one(self, token):
         """BitLlama::forward_one (llama.rs:201-271): one token at the current position;
@@ -385,7 +386,7 @@ class BitLlamaHip:
         """One decode step with the position on the device: the token in next_id at
         position *d_pos through the blocks and the head, then the greedy pick
         (next_id, log[*d_pos + 1], ++*d_pos)."""
-        self._run(1, self.pos, self.d_pos, self.next_id)
+        self._run(1, max(self.pos, self._expect), self.d_pos, self.next_id)
         check(lib.btl_greedy_next(self.logits.data_ptr(), self.cfg.vocab, self.next_id.data_ptr(),
                                   self.d_pos.data_ptr(), self.log.data_ptr(), self.log.numel(), self._stream()))
 
@@ -401,7 +402,6 @@ class BitLlamaHip:
                 self._step_device()
         torch.cuda.synchronize(self.dev)
         self.graph = g
-        self._graph_until = max(1024, 2 * self.pos)
         return g
 
     def start_decode(self):
@@ -411,17 +411,13 @@ class BitLlamaHip:
             self.log[self.pos:self.pos + 1].copy_(self.next_id)
 
     def decode_steps(self, n, use_graph=True):
-        """n greedy steps on the device; the tokens accumulate in self.log.  No host
-        synchronisation in between, but for a new capture of the step when the
-        position has doubled since the last one, and is 1024 at least: the launches
-        of the attention are chosen by it."""
+        """n greedy steps on the device, no host synchronisation in between; the
+        tokens accumulate in self.log."""
         if self.pos + n > self.cfg.max_seq:
             raise ValueError("%d steps from position %d overflow the cache of %d rows"
                              % (n, self.pos, self.cfg.max_seq))
         for _ in range(n):
             if use_graph and self.graph is not None:
-                if self.pos >= self._graph_until:
-                    self.capture_decode()
                 self.graph.replay()
             else:
                 self._step_device()
@@ -437,6 +433,8 @@ class BitLlamaHip:
         self.start_decode()
         if max_tokens > 1:
             if use_graph:
+                # the attention's launches are chosen once for all the steps: by their middle
+                self._expect = start + max_tokens // 2
                 self.capture_decode()
             self.decode_steps(max_tokens - 1, use_graph=use_graph)
         torch.cuda.synchronize(self.dev)

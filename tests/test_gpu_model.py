@@ -815,27 +815,26 @@ def test_decoder_prefill_equals_token_by_token(cfg_cls):
         assert torch.equal(a.caches[li].k_scale, b.caches[li].k_scale)
 
 
-def test_decoder_steps_over_a_new_capture():
-    # the step is captured anew at position 1024 (then where the position has doubled)
+def test_decoder_steps_launch_by_their_position():
+    # the captured step takes the attention's launches by the middle of the steps that
+    # replay it; the same tokens whichever it takes
     cfg = TinyA()
     cfg.max_seq = 2300
     w = tiny_weights(cfg, seed=5)
     prompt = np.random.default_rng(3).integers(0, cfg.vocab, 505)
-    logs = []
-    for use_graph in (True, False):
-        gm = gpu_model(cfg, w)
-        gm.prefill(prompt)
-        gm.greedy()
-        gm.start_decode()
-        if use_graph:
-            first = gm.capture_decode()
-            for n in (519, 1, 30):
-                gm.decode_steps(n)
-                assert (gm.graph is first) == (gm.pos <= 1024) and gm.d_pos.item() == gm.pos
-        else:
-            gm.decode_steps(550, use_graph=False)
-        logs.append(gm.log[505:1056].clone())
-    assert gm.pos == 1055 and torch.equal(*logs)
+    gm = gpu_model(cfg, w)
+    two = []
+
+    def captured():
+        two.append(any("k_attn_combine1" in f for f in launched(gm._step_device)))
+
+    gm.capture_decode, capture = captured, gm.capture_decode
+    for n in (100, 652, 660):  # its middle at 555, 831 and 835
+        gm.generate(prompt, n)
+    assert two == [False, False, True]
+    gm.capture_decode = capture
+    got = [gm.generate(prompt, 660, use_graph=g) for g in (True, False)]
+    assert len(got[0]) == 660 and np.array_equal(*got)
 
 
 @pytest.mark.parametrize("use_graph", [False, True])
